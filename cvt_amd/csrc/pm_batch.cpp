@@ -63,6 +63,12 @@ struct pm_batch {
   size_t arena_bytes = 0;
   long long nitems = 0;              // tile blocks of all pairs
   pm::BatchShape shape;
+  // the propagate takes wide tiles when every pair's fit a CU, the batch
+  // has one for every CU, and the shape is the default or has 8 tile rows
+  bool wide_ok = false;
+  bool shape_set = false;            // by pm_batch_set_tuning / _autotune
+  long long nwide = 0;               // wide tiles of all pairs
+  float max_dmax = 0.0f;             // largest disparity_max
   bool ran = false;
   int cur = 0;                       // plane field of the last run's result
   bool counted = false;              // the last run counted errors
@@ -141,13 +147,27 @@ int check_params(pm_batch* b, const pm_params* p) {
 // descriptor fields that depend on the tile rows: blocks per row and each
 // pair's first block in the batch sequence
 void number_blocks(pm_batch* b) {
-  long long item = 0;
+  long long item = 0, wide = 0;
   for (pm::BatchPair& P : b->host) {
     P.nbx = (P.g.W + 63) / 64;
     P.item0 = item;
+    P.wide0 = wide;
     item += pm::batch_blocks(P.g.W, P.g.H, b->shape.rows);
+    wide += pm::wide_tiles(P.g.W, P.g.H);
   }
   b->nitems = item;
+  b->nwide = wide;
+  b->wide_ok = pm::wide_fits(b->prm.radius, b->prm.cost_kind, b->max_dmax,
+                             b->maxW) &&
+               wide >= pm::kWideMinTiles;
+}
+
+bool use_wide(const pm_batch* b) {
+  return b->wide_ok && (!b->shape_set || b->shape.rows == 8);
+}
+
+size_t wide_lds(const pm_batch* b) {
+  return pm::wide_lds_bytes(b->prm.radius, b->prm.cost_kind, b->max_dmax);
 }
 
 int upload(pm_batch* b) {
@@ -209,7 +229,8 @@ int enqueue_proposal_init(pm_batch* b, hipStream_t st) {
 int enqueue_setup(pm_batch* b, hipStream_t st) {
   const size_t lds = tile_lds(b, b->shape.rows);
   PB_HIP(b, pm::launch_prepare_batch(st, b->dev, b->n, b->maxW, b->maxH,
-                                     b->prm.radius, b->prm.color_weight));
+                                     b->prm.radius, b->prm.color_weight,
+                                     b->prm.cost_kind, b->prm.cost_weight));
   if (b->net) {
     int rc;
     if ((rc = enqueue_proposal_init(b, st))) return rc;
@@ -229,6 +250,12 @@ int enqueue_propagate(pm_batch* b, hipStream_t st, int view, int cur,
                       int iter) {
   PB_HIP(b, pm::launch_viewbuf_clear_batch(st, b->dev, b->n, b->maxW,
                                            b->maxH, view));
+  if (use_wide(b)) {
+    PB_HIP(b, pm::launch_propagate_batch_wide(
+                  st, b->dev, b->n, b->nwide, view, cur, iter,
+                  b->prm.cost_kind, wide_lds(b), b->shape.workgroups));
+    return PM_OK;
+  }
   PB_HIP(b, pm::launch_propagate_batch(st, b->dev, b->n, b->nitems, view,
                                        cur, iter, b->prm.cost_kind,
                                        tile_lds(b, b->shape.rows), b->shape));
@@ -260,6 +287,8 @@ int allow_shape(pm_batch* b, int rows) {
   if (resident < 1)
     return fail(b, PM_ERR_ARG, "tile rows %d at radius %d do not fit a CU",
                 rows, b->prm.radius);
+  if (b->wide_ok)
+    PB_HIP(b, pm::batch_allow_wide(b->prm.cost_kind, wide_lds(b)));
   return PM_OK;
 }
 
@@ -359,10 +388,11 @@ int pm_batch_create(const pm_params* p, const pm_batch_pair* pairs, int n,
   for (int i = 0; i < n; ++i) {
     const size_t W = pairs[i].width, H = pairs[i].height, np = W * H;
     off[i] = total;
-    total += 2 * align_up(pm::tex_stride((int)W) * H * 2 * sizeof(float4));
+    total += 2 * align_up(pm::tex_bytes((int)W, (int)H));
     total += 2 * align_up(np);                        // sign bits
     total += 4 * align_up(np * sizeof(float4));       // plane fields
     total += 2 * align_up(np * sizeof(unsigned long long));
+    total += 2 * align_up(np * pm::kFlatCosts * sizeof(float));
     total += align_up(np * sizeof(float4));           // checked
     total += align_up(np * sizeof(float));            // disparity
     total += align_up(3 * sizeof(unsigned long long));
@@ -395,7 +425,7 @@ int pm_batch_create(const pm_params* p, const pm_batch_pair* pairs, int n,
     P.g.cost_weight = p->cost_weight;
     for (int v = 0; v < 2; ++v)
       P.v[v].tex = reinterpret_cast<float4*>(
-          take(pm::tex_stride(q.width) * H * 2 * sizeof(float4)));
+          take(pm::tex_bytes(q.width, q.height)));
     for (int v = 0; v < 2; ++v)
       P.v[v].sgn = reinterpret_cast<uint8_t*>(take(np));
     for (int v = 0; v < 2; ++v)
@@ -404,6 +434,9 @@ int pm_batch_create(const pm_params* p, const pm_batch_pair* pairs, int n,
     for (int v = 0; v < 2; ++v)
       P.vbuf[v] = reinterpret_cast<unsigned long long*>(
           take(np * sizeof(unsigned long long)));
+    for (int v = 0; v < 2; ++v)
+      P.flat[v] = reinterpret_cast<float*>(
+          take(np * pm::kFlatCosts * sizeof(float)));
     P.checked = reinterpret_cast<float4*>(take(np * sizeof(float4)));
     P.disp = reinterpret_cast<float*>(take(np * sizeof(float)));
     P.counts = reinterpret_cast<unsigned long long*>(
@@ -417,6 +450,7 @@ int pm_batch_create(const pm_params* p, const pm_batch_pair* pairs, int n,
     P.dmax = q.disparity_max;
     b->maxW = std::max(b->maxW, q.width);
     b->maxH = std::max(b->maxH, q.height);
+    b->max_dmax = std::max(b->max_dmax, q.disparity_max);
   }
   number_blocks(b);
   return upload(b);
@@ -575,7 +609,9 @@ int pm_batch_set_tuning(pm_batch* b, const pm_batch_tuning* t) {
   PB_HIP(b, hipSetDevice(b->prm.device));
   int rc;
   if ((rc = allow_shape(b, t->tile_rows))) return rc;
-  if (t->tile_rows != b->shape.rows || t->workgroups != b->shape.workgroups) {
+  if (t->tile_rows != b->shape.rows ||
+      t->workgroups != b->shape.workgroups || !b->shape_set) {
+    b->shape_set = true;
     b->shape.rows = t->tile_rows;
     b->shape.workgroups = t->workgroups;
     b->tuned_ms = 0.0f;

@@ -53,6 +53,8 @@ struct pm_ctx {
   DevBuf tex[2], sgn[2];
   DevBuf state[2][2];   // [view][ping-pong]
   DevBuf vbuf[2];       // vbuf[0]: filled by the left view, vbuf[1]: right
+  DevBuf flat[2];       // costs of the cleared smooth field's proposal
+  bool costs_known[2] = {};  // the plane field's cost channel can be trusted
   DevBuf checked;       // LR-checked left field
   DevBuf scratch4;      // W*H float4 (host transfers, normals)
   DevBuf scratch4b;     // W*H float4
@@ -191,13 +193,15 @@ int alloc_pair(pm_ctx* c, int W, int H, int channels) {
   int rc;
   for (int v = 0; v < 2; ++v) {
     if ((rc = ensure(c, c->img[v], n * channels * sizeof(float)))) return rc;
-    if ((rc = ensure(c, c->tex[v], (size_t)pm::tex_stride(W) * H * 2 *
-                                       sizeof(float4))))
+    if ((rc = ensure(c, c->tex[v], pm::tex_bytes(W, H))))
       return rc;
     if ((rc = ensure(c, c->sgn[v], n))) return rc;
     for (int k = 0; k < 2; ++k)
       if ((rc = ensure(c, c->state[v][k], n * sizeof(float4)))) return rc;
     if ((rc = ensure(c, c->vbuf[v], n * sizeof(unsigned long long))))
+      return rc;
+    if (c->prm.smoothing == PM_SMOOTH_NONE &&
+        (rc = ensure(c, c->flat[v], n * pm::kFlatCosts * sizeof(float))))
       return rc;
   }
   if ((rc = ensure(c, c->checked, n * sizeof(float4)))) return rc;
@@ -291,6 +295,8 @@ int set_images(pm_ctx* c, const float* l, const float* r, int W, int H,
 
 // bilateral weights + gradients of both views (PMHuberStereo.cpp:445-450)
 int prepare_views(pm_ctx* c, hipStream_t st = nullptr) {
+  PM_HIP(c, pm::launch_clear_wild(st ? st : c->stream, c->geo,
+                                  view_bufs(c, 0), view_bufs(c, 1)));
   for (int v = 0; v < 2; ++v)
     PM_HIP(c, pm::launch_prepare(st ? st : c->stream, c->geo,
                                  static_cast<const float*>(c->img[v].ptr),
@@ -416,7 +422,7 @@ static_assert(kSplitParts >= 2, "the split schedule needs two bands");
 constexpr int kBandReach = 5;
 
 int block_rows(const pm_ctx* c) {
-  return (c->geo.H + pm::kBlockRows - 1) / pm::kBlockRows;
+  return (c->geo.H + pm::kBandRows - 1) / pm::kBandRows;
 }
 
 // true when every band of the split schedule gets a block row; the
@@ -433,8 +439,8 @@ int band_first(const pm_ctx* c, int k) {
 
 // image rows [*r0, *r1) of band k
 void band_rows(const pm_ctx* c, int k, int* r0, int* r1) {
-  *r0 = band_first(c, k) * pm::kBlockRows;
-  *r1 = std::min(c->geo.H, band_first(c, k + 1) * pm::kBlockRows);
+  *r0 = band_first(c, k) * pm::kBandRows;
+  *r1 = std::min(c->geo.H, band_first(c, k + 1) * pm::kBandRows);
 }
 
 hipStream_t band_stream(const pm_ctx* c, int k) {
@@ -492,8 +498,8 @@ int propagate_split(pm_ctx* c, const pm::PropagateArgs& a, int view,
     int r0, r1;
     band_rows(c, k, &r0, &r1);
     pm::Geometry g = c->geo;
-    g.by0 = band_first(c, k);
-    g.nby = band_first(c, k + 1) - g.by0;
+    g.band0 = band_first(c, k);
+    g.bands = band_first(c, k + 1) - g.band0;
     const hipStream_t st = band_stream(c, k);
     PM_HIP(c, pm::launch_viewbuf_clear_rows(st, c->geo, vb, r0, r1 - r0));
     PM_HIP(c, pm::launch_propagate(st, g, a, counters, c->prop_lds_floor));
@@ -568,7 +574,9 @@ float theta_after(const pm_ctx* c, int i, float theta) {
 
 // pmhstereo_propagate_view for the left then the right view, each followed
 // by its PM-Huber smoothing (PMHuberStereo.cpp:530-578)
-int one_iteration(pm_ctx* c, unsigned long long* counters, bool split) {
+// first: the first iteration of its pm_iterate call
+int one_iteration(pm_ctx* c, unsigned long long* counters, bool split,
+                  bool first) {
   const int cur = c->cur, nxt = 1 - c->cur;
   unsigned long long* vbL = static_cast<unsigned long long*>(c->vbuf[0].ptr);
   unsigned long long* vbR = static_cast<unsigned long long*>(c->vbuf[1].ptr);
@@ -579,8 +587,11 @@ int one_iteration(pm_ctx* c, unsigned long long* counters, bool split) {
   a.theta = huber ? theta * (depthmap_mode(c) ? kDepthThetaScale : kThetaScale)
                  : 0.0f;
   a.iter = c->iteration;
+  a.flat_known = first ? 0 : 1;
   int rc;
 
+  a.costs_known = c->costs_known[0];
+  a.flat_cost = huber ? nullptr : static_cast<float*>(c->flat[0].ptr);
   a.self = view_bufs(c, 0);
   a.other = view_bufs(c, 1);
   a.old = state_ptr(c, 0, cur);
@@ -594,6 +605,8 @@ int one_iteration(pm_ctx* c, unsigned long long* counters, bool split) {
   if (huber && (rc = smooth_after(c, 0, state_ptr(c, 0, nxt), theta, split)))
     return rc;
 
+  a.costs_known = c->costs_known[1];
+  a.flat_cost = huber ? nullptr : static_cast<float*>(c->flat[1].ptr);
   a.self = view_bufs(c, 1);
   a.other = view_bufs(c, 0);
   a.old = state_ptr(c, 1, cur);
@@ -610,6 +623,7 @@ int one_iteration(pm_ctx* c, unsigned long long* counters, bool split) {
   if (huber) {
     c->theta = theta_after(c, c->iteration, c->theta);
   }
+  c->costs_known[0] = c->costs_known[1] = true;
   c->cur = nxt;
   c->iteration += 1;
   return PM_OK;
@@ -632,7 +646,7 @@ int iterate_n(pm_ctx* c, int n, unsigned long long* counters) {
   }
   if (split && (rc = split_rebase(c))) return rc;
   for (int i = 0; i < n; ++i)
-    if ((rc = one_iteration(c, counters, split))) break;
+    if ((rc = one_iteration(c, counters, split, i == 0))) break;
   if (split) {
     // joined even after a failed launch, so that no work is left behind
     // unordered on the other streams: each records how far it has got and
@@ -800,6 +814,7 @@ void pm_destroy(pm_ctx* c) {
     release(c->state[v][0]);
     release(c->state[v][1]);
     release(c->vbuf[v]);
+    release(c->flat[v]);
     release(c->dt[v]);
     release(c->smooth[v]);
     release(c->rofb[v].nd);
@@ -862,6 +877,7 @@ int pm_setup(pm_ctx* c) {
   if ((rc = huber_setup(c))) return rc;
   c->cur = 0;
   c->iteration = 0;
+  c->costs_known[0] = c->costs_known[1] = true;
   c->ready = true;
   c->last_pp = -1;
   return PM_OK;
@@ -935,6 +951,7 @@ int pm_setup_proposal_views(pm_ctx* c, pm_net* net, int views) {
   if ((rc = huber_setup(c))) return rc;
   c->cur = 0;
   c->iteration = 0;
+  c->costs_known[0] = c->costs_known[1] = true;
   c->ready = true;
   c->last_pp = -1;
   return PM_OK;
@@ -974,6 +991,7 @@ int pm_setup_prior(pm_ctx* c, const float* disparity, const float* normals) {
   PM_HIP(c, hipStreamSynchronize(c->stream));  // host inputs may be freed
   c->cur = 0;
   c->iteration = 0;
+  c->costs_known[0] = c->costs_known[1] = true;
   c->ready = true;
   c->last_pp = -1;
   return PM_OK;
@@ -1032,6 +1050,7 @@ int pm_set_planes(pm_ctx* c, int view, const float* in, int iteration) {
     return rc;
   if (!in) return fail(c, PM_ERR_ARG, "in is NULL");
   if (iteration < 0) return fail(c, PM_ERR_ARG, "negative iteration");
+  c->costs_known[view] = false;  // whatever the caller's cost channel holds
   if ((rc = to_device(c, state_ptr(c, view, c->cur), in,
                       c->geo.npix * sizeof(float4))))
     return rc;

@@ -31,10 +31,28 @@ __host__ __device__ inline int tex_stride(int W) {
   return W + kTexPadL + kTexPadR;
 }
 
+// After the two planes of a view's texel buffer: the colours again as
+// packed 12-byte records (r, g, b), rows padded the same way, so that one
+// lane's neighbouring texels are one run of bytes; then one word that is
+// nonzero when the image is not tame (pm_engine.hip says what that is),
+// cleared by launch_clear_wild and set by launch_prepare.
+__host__ __device__ inline float* packed_colours(float4* tex, int TS, int H) {
+  return reinterpret_cast<float*>(tex + (size_t)TS * H * 2);
+}
+__host__ __device__ inline uint32_t* wild_word(float4* tex, int TS, int H) {
+  return reinterpret_cast<uint32_t*>(packed_colours(tex, TS, H) +
+                                     (size_t)TS * H * 3);
+}
+__host__ __device__ inline size_t tex_bytes(int W, int H) {
+  return (size_t)tex_stride(W) * H * 44 + sizeof(uint32_t);
+}
+
 // work-group tiles of the cost-evaluating kernels: kBlockCols x kBlockRows
 // pixels
 constexpr int kBlockCols = 64;
 constexpr int kBlockRows = 4;
+// a propagate launch covers whole bands of this many rows
+constexpr int kBandRows = 8;
 
 // candidate cost of the plane-evaluating kernels: what the reference's
 // `#define patch_eval` (pmhstereo.cl:753) selects
@@ -47,9 +65,9 @@ struct Geometry {
   int W = 0, H = 0, R = 0;
   int TS = 0;  // texel row stride in records, tex_stride(W)
   size_t npix = 0;
-  // a launch covers the block rows [by0, by0 + nby) of the image
-  // (nby = 0: all of them)
-  int by0 = 0, nby = 0;
+  // a propagate covers the bands [band0, band0 + bands) of kBandRows image
+  // rows (bands = 0: all of them)
+  int band0 = 0, bands = 0;
   // CENSUS_COLOR_WEIGHT: bilateral weight sum, census cost and KLT step
   float color_weight = 12.0f;
   int cost_kind = kCostCensus;
@@ -59,7 +77,22 @@ struct Geometry {
   // red-black propagate pass: -1 = every pixel (the reference's Jacobi
   // sweep), 0 / 1 = only the pixels with (x + y) & 1 equal to it
   int color = -1;
+
+  __host__ __device__ int row_end() const {
+    const int e = (band0 + bands) * kBandRows;
+    return bands > 0 && e < H ? e : H;
+  }
 };
+
+// window of the other view's columns a propagate's tile block keeps in LDS:
+// from `left` columns left of the block's first, `cols` columns (0: none)
+struct Window {
+  int left = 0, cols = 0;
+};
+
+// before the launch_prepare of the two views
+hipError_t launch_clear_wild(hipStream_t st, const Geometry& g, ViewBufs a,
+                             ViewBufs b);
 
 hipError_t launch_prepare(hipStream_t st, const Geometry& g, const float* img,
                           int channels, int stride, ViewBufs v);
@@ -103,7 +136,19 @@ struct PropagateArgs {
   // red-black pass 1 (Geometry::color == 1): the pass-0 pixels' new planes,
   // read instead of `old` for neighbours of colour 0 (may alias `out`)
   const float4* fresh = nullptr;
+  // the cost channel of `old` holds its planes' costs (of this cost kind,
+  // as an evaluation without an early exit gives them, or NaN, or the 1.0
+  // of the census exit)
+  int costs_known = 0;
+  // without a smooth field: kFlatCosts floats per pixel for the cost of the
+  // cleared field's proposal, written (flat_known = 0) or read; may be null
+  float* flat_cost = nullptr;
+  int flat_known = 0;
 };
+
+// floats per pixel of PropagateArgs::flat_cost: the cost and, for the
+// census cost, the quotient its early exit compares
+constexpr int kFlatCosts = 2;
 
 // counters (optional, 2 x u64): cost taps and KLT taps evaluated, counted
 // with the reference's per-tap early exit.  lds_floor: the work-groups ask
@@ -113,6 +158,14 @@ hipError_t launch_propagate(hipStream_t st, const Geometry& g,
                             const PropagateArgs& a,
                             unsigned long long* counters = nullptr,
                             size_t lds_floor = 0);
+
+// The propagate's wide tile (pm_engine.hip): its LDS at a patch radius, cost
+// kind and disparity range, whether that fits a CU, the tiles of an image,
+// and the tiles from which on it is used (one per CU).
+size_t wide_lds_bytes(int R, int cost_kind, float dmax);
+bool wide_fits(int R, int cost_kind, float dmax, int maxW);
+long long wide_tiles(int W, int H);
+constexpr int kWideMinTiles = 256;
 
 hipError_t launch_scatter(hipStream_t st, const Geometry& g,
                           const float4* states, int lr,
@@ -198,6 +251,7 @@ struct BatchPair {
   ViewBufs v[2];
   float4* state[2][2];      // [view][ping-pong]
   unsigned long long* vbuf[2];
+  float* flat[2];           // PropagateArgs::flat_cost of each view
   float4* checked;          // LR-checked left field
   float* disp;              // disparity out (W x H)
   const float* img[2];      // input images, `stride` floats per row
@@ -207,6 +261,7 @@ struct BatchPair {
   float dmax;
   int nbx;                  // tile blocks per row (64 columns each)
   long long item0;          // first tile block of the pair in the batch
+  long long wide0;          // first wide tile of the pair in the batch
 };
 
 // tile blocks of 64 x rows pixels of a W x H image
@@ -228,7 +283,7 @@ constexpr int kBatchRowChoices[3] = {2, 4, 8};
 // bound the pairs' sizes
 hipError_t launch_prepare_batch(hipStream_t st, const BatchPair* pairs,
                                 int npairs, int maxW, int maxH, int R,
-                                float cw);
+                                float cw, int cost_kind, float kw);
 hipError_t launch_viewbuf_clear_batch(hipStream_t st, const BatchPair* pairs,
                                       int npairs, int maxW, int maxH,
                                       int view);
@@ -241,6 +296,13 @@ hipError_t launch_propagate_batch(hipStream_t st, const BatchPair* pairs,
                                   int npairs, long long nitems, int view,
                                   int cur, int iter, int cost_kind,
                                   size_t lds, BatchShape shape);
+// the same with wide tiles (nitems of them), lds for the pair that needs
+// most; batch_allow_wide before a capture
+hipError_t launch_propagate_batch_wide(hipStream_t st, const BatchPair* pairs,
+                                       int npairs, long long nitems, int view,
+                                       int cur, int iter, int cost_kind,
+                                       size_t lds, int workgroups);
+hipError_t batch_allow_wide(int cost_kind, size_t lds);
 // pp: 0 none, 1 LR check, 2 LR check + fill (pm_postproc)
 hipError_t launch_postprocess_batch(hipStream_t st, const BatchPair* pairs,
                                     int npairs, int maxW, int maxH, int cur,
