@@ -64,7 +64,7 @@ struct pm_batch {
   long long nitems = 0;              // tile blocks of all pairs
   pm::BatchShape shape;
   // the propagate takes wide tiles when every pair's fit a CU, the batch
-  // has one for every CU, and the shape is the default or has 8 tile rows
+  // has enough of them, and the shape is the default or has 8 tile rows
   bool wide_ok = false;
   bool shape_set = false;            // by pm_batch_set_tuning / _autotune
   long long nwide = 0;               // wide tiles of all pairs
@@ -159,7 +159,7 @@ void number_blocks(pm_batch* b) {
   b->nwide = wide;
   b->wide_ok = pm::wide_fits(b->prm.radius, b->prm.cost_kind, b->max_dmax,
                              b->maxW) &&
-               wide >= pm::kWideMinTiles;
+               wide >= pm::wide_min_tiles(b->prm.radius);
 }
 
 bool use_wide(const pm_batch* b) {

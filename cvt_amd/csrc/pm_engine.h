@@ -161,11 +161,11 @@ hipError_t launch_propagate(hipStream_t st, const Geometry& g,
 
 // The propagate's wide tile (pm_engine.hip): its LDS at a patch radius, cost
 // kind and disparity range, whether that fits a CU, the tiles of an image,
-// and the tiles from which on it is used (one per CU).
+// and the tiles from which on it is used.
 size_t wide_lds_bytes(int R, int cost_kind, float dmax);
 bool wide_fits(int R, int cost_kind, float dmax, int maxW);
 long long wide_tiles(int W, int H);
-constexpr int kWideMinTiles = 256;
+int wide_min_tiles(int R);
 
 hipError_t launch_scatter(hipStream_t st, const Geometry& g,
                           const float4* states, int lr,

@@ -2177,12 +2177,17 @@ size_t wide_lds_bytes(int R, int cost_kind, float dmax) {
                         window_of(R, dmax, 1).cols);
 }
 
-// The wide tile fits when its window and tiles fit a CU's LDS, and pays
-// when the image gives every CU at least one.  Measured against the 64 x 4
-// tiles without a window (8 iterations or the case's own): 1280 x 720
-// colour+gradient (450 tiles, 900 in all) 51.2 -> 45.2 ms, 1242 x 375
-// (470 tiles) 38.2 -> 33.9, 640 x 480 (300) 20.0 -> 18.7, 320 x 240 (90)
-// 5.0 -> 7.3.
+// The wide tile fits when its window and tiles fit a CU's LDS; it pays
+// (wide_min_tiles) when the image has enough of them: a CU holds one, so an
+// image of 260 tiles takes two rounds with the second nearly empty, and the
+// smaller the patch the less the window saves per tile staged.  Time against
+// the 64 x 4 tiles without a window, plain PatchMatch:
+//   tiles    260   300   350   400   512   650
+//   R = 2   1.11  1.04  1.05  1.01  0.96  0.96
+//   R = 4   1.09  0.99  0.98  0.95  0.91  0.91
+//   R = 5   1.07  0.95  0.96  0.94  0.90  0.90
+int wide_min_tiles(int R) { return R >= 4 ? 300 : 448; }
+
 bool wide_fits(int R, int cost_kind, float dmax, int maxW) {
   return dmax < 4096.0f && maxW < (1 << 23) &&
          wide_lds_bytes(R, cost_kind, dmax) <= kLdsPerCu;
@@ -2198,7 +2203,7 @@ static hipError_t launch_propagate_kind(hipStream_t st, const Geometry& g,
                                         unsigned long long* counters,
                                         size_t lds_floor) {
   if (!kRB && !counters && wide_fits(g.R, kKind, a.dmax, g.W) &&
-      wide_tiles(g.W, g.H) >= kWideMinTiles)
+      wide_tiles(g.W, g.H) >= wide_min_tiles(g.R))
     return launch_propagate_tile<kKind, false, false, kWideRows,
                                  kWideCols / kTX, true>(
         st, g, a, counters, wide_lds_bytes(g.R, kKind, a.dmax),

@@ -1,5 +1,6 @@
 """The propagate's wide tiles (128 x 8 pixels with a window of the other
-view in LDS, taken by images of at least 256 of them), the tame and the
+view in LDS, taken by images of at least 448 of them, 300 from a patch
+radius of 4 on), the tame and the
 general loops, and the costs it does not evaluate again, bit for bit
 against the oracle or against the calls that evaluate them."""
 import numpy as np
@@ -33,11 +34,11 @@ def check(oracle, L, R, r, dmax, iters, kind, kw):
 # partial tiles on both sides, a window wider than the image, windows of
 # almost no range, two rows of very many tiles, the largest patch that fits
 @pytest.mark.parametrize("W,H,C,r,dmax,iters,kind", [
-    (2053, 131, 4, 3, 200.0, 2, CG),
+    (2053, 219, 4, 3, 200.0, 1, CG),
     (1153, 263, 1, 5, 17.0, 2, CENSUS),
-    (2049, 129, 4, 1, 3.5, 3, CENSUS),
-    (16389, 9, 1, 2, 30.0, 2, CG),
-    (1031, 251, 4, 8, 12.0, 1, CENSUS),
+    (2049, 219, 4, 1, 3.5, 3, CENSUS),
+    (28677, 9, 1, 2, 30.0, 2, CG),
+    (1031, 275, 4, 8, 12.0, 1, CENSUS),
 ])
 def test_wide_tiles_bitexact(oracle, synth, W, H, C, r, dmax, iters, kind):
     L, R, _ = synth.make_pair(W, H, cells=9, dmax=min(dmax, 60.0),
@@ -49,7 +50,7 @@ def test_wide_tiles_bitexact(oracle, synth, W, H, C, r, dmax, iters, kind):
 @pytest.mark.parametrize("value", [1e5, -1e-30, -0.0])
 @pytest.mark.parametrize("kind", [CENSUS, CG])
 def test_untame_images_bitexact(oracle, synth, value, kind):
-    L, R, _ = synth.make_pair(1030, 250, cells=9, dmax=30.0, channels=4,
+    L, R, _ = synth.make_pair(1030, 400, cells=9, dmax=30.0, channels=4,
                               seed=5)
     for img, x, y in ((L, 400, 100), (R, 611, 37)):
         img[y:y + 3, x:x + 4, 1] = value
@@ -60,7 +61,7 @@ def test_untame_images_bitexact(oracle, synth, value, kind):
 def test_iterating_in_one_call_and_in_several(synth, kind):
     """the flat proposal's cost, kept within a call, and the plane costs,
     kept from one iteration to the next"""
-    L, R, _ = synth.make_pair(1100, 240, cells=9, dmax=30.0, channels=4,
+    L, R, _ = synth.make_pair(1100, 400, cells=9, dmax=30.0, channels=4,
                               seed=6)
     with cvt_amd.Context(radius=3, disparity_max=30.0, cost_kind=kind) as ctx:
         one = run(ctx, L, R, 3)
@@ -70,7 +71,7 @@ def test_iterating_in_one_call_and_in_several(synth, kind):
         assert same(ctx.planes(0), one[0]) and same(ctx.planes(1), one[1])
 
 
-@pytest.mark.parametrize("W,H", [(90, 40), (1100, 240)])
+@pytest.mark.parametrize("W,H", [(90, 40), (1100, 400)])
 @pytest.mark.parametrize("kind", [CENSUS, CG])
 def test_a_callers_cost_channel_is_not_trusted(synth, W, H, kind):
     L, R, _ = synth.make_pair(W, H, cells=6, dmax=20.0, channels=4, seed=7)
