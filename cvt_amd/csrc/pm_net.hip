@@ -4,6 +4,7 @@
 // same instruction), and the pooling, gradient routing, loss, Adam and input
 // packing kernels of a U-Net training step.
 #include <algorithm>
+#include <cstdint>
 
 #include "pm_net_kernels.h"
 
@@ -11,7 +12,9 @@ namespace pm {
 namespace net {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+typedef __attribute__((__vector_size__(16))) uint32_t u32x4;
 
 #define NET_LAUNCH(kernel, grid, block, lds, st, ...)               \
   do {                                                              \
@@ -31,111 +34,216 @@ __device__ __forceinline__ bf16x8 zero8() {
   return z;
 }
 
-// ---------------------------------------------------------------------
-// convolution: a work-group is one wavefront computing 64 output pixels x
-// 16 kNT output channels as 4 x kNT tiles of 16 x 16.  Per K step of 32 a lane
-// holds the A operand of its tile row (pixel) and k-group (8 consecutive
-// k: one tap, 8 channels, one 16-byte load from NHWC) and the B operand
-// of its tile column (output channel: 8 consecutive k of its weight row).
-// The accumulator of a lane holds rows 4 g .. 4 g + 3, column lane % 16.
-// ---------------------------------------------------------------------
-constexpr int kConvPix = 64;
+// Every convolution multiplies weights (rows: output channels) by pixels
+// (columns): lane l ends with channels 4 (l / 16) .. + 3 of pixel l % 16, so
+// it writes 8 bytes (16 in fp32) where the other order writes 2.  vec: the
+// output rows are aligned for that (an output given by a caller may not be).
+__device__ __forceinline__ f32x4 conv_bias4(const ConvArgs& a, int co) {
+  f32x4 b = {0.f, 0.f, 0.f, 0.f};
+  if (a.bias) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b[j] = a.bias[std::min(co + j, a.cout - 1)];
+  }
+  return b;
+}
 
-// kNT column tiles of 16 output channels per wavefront: 2 (32 channels)
-// or 4 (64, when the padded output count is a multiple of 64, which
-// halves the A loads per matrix-core op)
-template <int kNT>
-__global__ void __launch_bounds__(64) k_conv(ConvArgs a) {
-  const int lane = threadIdx.x;
+__device__ __forceinline__ void conv_store4(const ConvArgs& a, size_t p,
+                                            int co, const f32x4& acc,
+                                            const f32x4& bias, bool vec) {
+  if (co >= a.cout) return;
+  float v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    v[j] = acc[j] + bias[j];
+    if (a.relu) v[j] = fmaxf(v[j], 0.0f);
+  }
+  if (vec) {
+    if (a.yf) {
+      *reinterpret_cast<float4*>(a.yf + p * a.ys + co) =
+          make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+      bf16x4 o;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = (bf16)v[j];
+      *reinterpret_cast<bf16x4*>(a.y + p * a.ys + co) = o;
+    }
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (co + j >= a.cout) continue;
+    if (a.yf)
+      a.yf[p * a.ys + co + j] = v[j];
+    else
+      a.y[p * a.ys + co + j] = (bf16)v[j];
+  }
+}
+
+static bool conv_vec_store(const ConvArgs& a) {
+  const uintptr_t mask = a.yf ? 15 : 7;
+  const uintptr_t ptr = reinterpret_cast<uintptr_t>(
+      a.yf ? static_cast<const void*>(a.yf) : static_cast<const void*>(a.y));
+  return a.ys % 4 == 0 && a.cout % 4 == 0 && (ptr & mask) == 0;
+}
+
+// ---------------------------------------------------------------------
+// lattice convolution: any dilation, any channels.  The pixels a dilated
+// kernel couples are a lattice (every dil-th column and row), so a
+// work-group takes a tile of 16 x kMT lattice pixels with its one-pixel rim,
+// stages all their input channels in LDS once and shares them among its
+// wavefronts, each of 16 kNT output channels.  Per K step of 32 a lane reads
+// its pixel's 8 consecutive k (one tap, 8 channels) from there and its
+// weight row's from memory (L2), kDepth steps ahead: with one step at a
+// time the layers here are a chain of trips to L2.  An LDS pixel takes an
+// odd number of 16-byte pieces, so 16 neighbours hit distinct banks.
+// K is summed tap by tap, channels within a tap.
+// Against a gather of every operand from memory, one wavefront with 64
+// pixels x 64 channels: 128 -> 128 channels at 160 x 90, dilation 2 / 4 / 8,
+// 54 / 53 / 52 -> 18 / 18 / 20 us, at 40 x 30 50 -> 11; 112 -> 96 at 320 x 180
+// 61 -> 28; 8 -> 32 at 1280 x 720, whose bound is the 59 MB it writes, 46 -> 24.
+// The dilated layers at 160 x 90 are 960 wavefronts, fewer than the SIMDs.
+// ---------------------------------------------------------------------
+constexpr int kLatX = 16;
+
+static int lattice_pieces(int cin) { return cin / 8 | 1; }
+
+template <int kMT>
+static size_t lattice_lds(int cin) {
+  return ((kLatX + 2) * (kMT + 2) * lattice_pieces(cin) + 1) * sizeof(uint4);
+}
+
+template <int kMT, int kNT, int kDepth>
+__global__ void __launch_bounds__(512)
+k_conv_lattice(ConvArgs a, int tiles_x, int tiles_y, bool vec) {
+  constexpr int kRimX = kLatX + 2, kRimY = kMT + 2;
+  extern __shared__ uint4 smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row = lane & 15, grp = lane >> 4;
-  const int cin = a.c1 + a.c2;
-  const int kpad = conv_kpad(cin), kreal = 9 * cin;
-  const long npix = (long)a.N * a.H * a.W;
-  const long p0 = (long)blockIdx.x * kConvPix;
-  const int co0 = blockIdx.y * (16 * kNT);
+  const int cin = a.c1 + a.c2, P = cin / 8, stride = P | 1;
+  const int kpad = conv_kpad(cin), steps = kpad / 32;
   const int H2 = a.up2 ? (a.H + 1) >> 1 : a.H;
   const int W2 = a.up2 ? (a.W + 1) >> 1 : a.W;
-  int pn[4], py[4], px[4];
-  bool pv[4];
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const long p = p0 + mt * 16 + row;
-    pv[mt] = p < npix;
-    const long q = pv[mt] ? p : 0;
-    px[mt] = (int)(q % a.W);
-    const long t = q / a.W;
-    py[mt] = (int)(t % a.H);
-    pn[mt] = (int)(t / a.H);
-  }
-  f32x4 acc[4][kNT];
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bf16* wrow = a.w + (size_t)(co0 + row) * kpad;
-  // this lane's k = k0 + 8 grp as (tap, channel), advanced by 32 per step
-  int tap = (8 * grp) / cin, ci = (8 * grp) % cin;
-  for (int k0 = 0; k0 < kpad; k0 += 32) {
-    const int k = k0 + 8 * grp;
-    bf16x8 A[4];
-    if (k < kreal) {
-      const int dy = (tap / 3 - 1) * a.dil, dx = (tap % 3 - 1) * a.dil;
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
-        const int yy = py[mt] + dy, xx = px[mt] + dx;
-        A[mt] = zero8();
-        if (pv[mt] && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) {
-          if (ci < a.c1) {
-            A[mt] = load8(a.x1 +
-                          (((size_t)pn[mt] * a.H + yy) * a.W + xx) * a.c1 +
-                          ci);
-          } else {
-            const int y2 = a.up2 ? yy >> 1 : yy, x2 = a.up2 ? xx >> 1 : xx;
-            A[mt] = load8(a.x2 +
-                          (((size_t)pn[mt] * H2 + y2) * W2 + x2) * a.c2 +
-                          (ci - a.c1));
-          }
-        }
-      }
-    } else {
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) A[mt] = zero8();
-    }
-    bf16x8 B[kNT];
+  // tile, then the lattice's offset, then the image
+  int t = blockIdx.x;
+  const int lx0 = t % tiles_x * kLatX;
+  t /= tiles_x;
+  const int ly0 = t % tiles_y * kMT;
+  t /= tiles_y;
+  const int ox = t % a.dil;
+  t /= a.dil;
+  const int oy = t % a.dil, n = t / a.dil;
+  const int co0 = (blockIdx.y * (blockDim.x >> 6) + wave) * (16 * kNT);
+  const bool busy = co0 < conv_cpad(a.cout);
+
+  // this lane's weights, kDepth steps ahead
+  const bf16* wrow = a.w + (size_t)(busy ? co0 + row : 0) * kpad + 8 * grp;
+  u32x4 bw[kDepth][kNT];
+  int next = 0;
+  auto load = [&](u32x4 (&v)[kNT]) {
+    const int k = 32 * std::min(next, steps - 1);
 #pragma unroll
     for (int nt = 0; nt < kNT; ++nt)
-      B[nt] = load8(wrow + (size_t)nt * 16 * kpad + k);
+      v[nt] = *reinterpret_cast<const u32x4*>(wrow + nt * 16 * kpad + k);
+    ++next;
+  };
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+  for (int d = 0; d < kDepth; ++d) load(bw[d]);
+
+  for (int q = tid; q < kRimX * kRimY * P; q += blockDim.x) {
+    const int pix = q / P, g = q - pix * P;
+    const int r = pix / kRimX, c = pix - r * kRimX;
+    const int yy = (ly0 + r - 1) * a.dil + oy;
+    const int xx = (lx0 + c - 1) * a.dil + ox;
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) {
+      if (8 * g < a.c1) {
+        v = *reinterpret_cast<const uint4*>(
+            a.x1 + (((size_t)n * a.H + yy) * a.W + xx) * a.c1 + 8 * g);
+      } else {
+        const int y2 = a.up2 ? yy >> 1 : yy, x2 = a.up2 ? xx >> 1 : xx;
+        v = *reinterpret_cast<const uint4*>(
+            a.x2 + (((size_t)n * H2 + y2) * W2 + x2) * a.c2 +
+            (8 * g - a.c1));
+      }
+    }
+    smem[pix * stride + g] = v;
+  }
+  constexpr int kRim = kRimX * kRimY;
+  if (tid == 0) smem[kRim * stride] = make_uint4(0u, 0u, 0u, 0u);
+  __syncthreads();
+  if (!busy) return;
+
+  f32x4 acc[kMT][kNT];
+#pragma unroll
+  for (int mt = 0; mt < kMT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < kNT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // this lane's k as (tap, piece); from tap 9 on there are no real k, and
+  // the piece of zeros behind the window is read
+  int tap = grp / P, g = grp - tap * P;
+  const int step_tap = 4 / P, step_g = 4 - step_tap * P;
+  auto multiply = [&](const u32x4 (&w)[kNT]) {
+    const int ty = (tap * 11) >> 5;  // tap / 3 for the taps there are
+    const int at = (ty * kRimX + tap - 3 * ty + row) * stride + g;
+    const bool real = tap < 9;
+#pragma unroll
+    for (int mt = 0; mt < kMT; ++mt) {
+      const uint4 v =
+          smem[real ? at + mt * kRimX * stride : kRim * stride];
 #pragma unroll
       for (int nt = 0; nt < kNT; ++nt)
         acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            A[mt], B[nt], acc[mt][nt], 0, 0, 0);
-    ci += 32;
-    while (ci >= cin) {
-      ci -= cin;
-      ++tap;
+            __builtin_bit_cast(bf16x8, w[nt]), __builtin_bit_cast(bf16x8, v),
+            acc[mt][nt], 0, 0, 0);
+    }
+    g += step_g;
+    tap += step_tap + (g >= P ? 1 : 0);
+    g -= g >= P ? P : 0;
+  };
+  int s = 0;
+  for (; s + kDepth <= steps; s += kDepth) {
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d) {
+      multiply(bw[d]);
+      load(bw[d]);
+      __builtin_amdgcn_sched_barrier(0);  // or all loads come last
     }
   }
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int d = 0; d < kDepth - 1; ++d)
+    if (s + d < steps) multiply(bw[d]);
+
+  f32x4 bias[kNT];
 #pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) {
-      const int co = co0 + nt * 16 + row;
-      if (co >= a.cout) continue;
-      const float b = a.bias ? a.bias[co] : 0.0f;
+  for (int nt = 0; nt < kNT; ++nt)
+    bias[nt] = conv_bias4(a, co0 + nt * 16 + 4 * grp);
+  const int x = (lx0 + row) * a.dil + ox;
+  if (x >= a.W) return;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const long p = p0 + mt * 16 + 4 * grp + j;
-        if (p >= npix) continue;
-        float v = acc[mt][nt][j] + b;
-        if (a.relu) v = fmaxf(v, 0.0f);
-        if (a.yf)
-          a.yf[p * a.ys + co] = v;
-        else
-          a.y[p * a.ys + co] = (bf16)v;
-      }
-    }
+  for (int mt = 0; mt < kMT; ++mt) {
+    const int y = (ly0 + mt) * a.dil + oy;
+    if (y >= a.H) continue;
+    const size_t p = ((size_t)n * a.H + y) * a.W + x;
+#pragma unroll
+    for (int nt = 0; nt < kNT; ++nt)
+      conv_store4(a, p, co0 + nt * 16 + 4 * grp, acc[mt][nt], bias[nt], vec);
+  }
+}
+
+template <int kMT, int kNT, int kDepth, int kWaves>
+static hipError_t launch_lattice(hipStream_t st, const ConvArgs& a,
+                                 bool vec) {
+  const int lw = (a.W + a.dil - 1) / a.dil, lh = (a.H + a.dil - 1) / a.dil;
+  const int tiles_x = (lw + kLatX - 1) / kLatX, tiles_y = (lh + kMT - 1) / kMT;
+  const int groups = conv_cpad(a.cout) / (16 * kNT);
+  const int waves = std::min(groups, kWaves);
+  const size_t lds = lattice_lds<kMT>(a.c1 + a.c2);
+  if (lds > 65536) return hipErrorInvalidValue;
+  NET_LAUNCH((k_conv_lattice<kMT, kNT, kDepth>),
+             dim3((unsigned)((long)tiles_x * tiles_y * a.dil * a.dil * a.N),
+                  (unsigned)((groups + waves - 1) / waves)),
+             dim3(64 * waves), lds, st, a, tiles_x, tiles_y, vec);
 }
 
 // ---------------------------------------------------------------------
@@ -160,32 +268,56 @@ __device__ __forceinline__ int lds_slot(int g, int col) {
   return g ^ ((col >> 1) & 3);
 }
 
-template <int kNT>
+// kWalk: one chunk (32 input channels), the full-resolution layers, which
+// are bound by memory and latency: a work-group walks tiles (a run of them,
+// top to bottom, so that the two shared rows are in its L2), stages its
+// weights once and reads the next tile's window during this one's products.
+// With one tile per work-group nothing overlapped its fetch: 32 -> 32
+// channels at 1280 x 720 (59 MB in, 59 out) 62 -> 32 us, the head 46 -> 24.
+// With more chunks the weights of all have to stay in LDS, and walking was
+// the slower form (96 -> 32: 88 us without, 99 with).
+template <int kNT, bool kWalk>
 __device__ __forceinline__ void conv_lds_block(const ConvArgs& a, int tiles_x,
-                                               int tiles_y) {
+                                               int tiles_y, int tiles,
+                                               bool vec) {
   constexpr int kCO = 16 * kNT;
   constexpr int kWPieces = 9 * kCO * 4;
   constexpr int kAIters = (kWinPieces + 255) / 256;
   constexpr int kBIters = (kWPieces + 255) / 256;
   __shared__ uint4 sA[kWinPieces];
   __shared__ uint4 sB[kWPieces];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row = lane & 15, grp = lane >> 4;
-  int t = blockIdx.x;
-  const int tx = t % tiles_x;
-  t /= tiles_x;
-  const int ty = t % tiles_y, n = t / tiles_y;
-  const int x0 = tx * kTileX, y0 = ty * kTileY;
   const int co0 = blockIdx.y * kCO;
   const int cin = a.c1 + a.c2;
   const int kpad = conv_kpad(cin);
   const int H2 = a.up2 ? (a.H + 1) >> 1 : a.H;
   const int W2 = a.up2 ? (a.W + 1) >> 1 : a.W;
-  const int nchunks = cin / 32;
+  const int nchunks = kWalk ? 1 : cin / 32;
+  int t = blockIdx.x, t_end = t + 1;
+  if (kWalk) {
+    t = (int)((long)blockIdx.x * tiles / gridDim.x);
+    t_end = (int)((long)(blockIdx.x + 1) * tiles / gridDim.x);
+  }
+  int n, x0, y0;
+  auto place = [&](int tile) {
+    if (kWalk) {  // top to bottom first
+      y0 = (tile % tiles_y) * kTileY;
+      tile /= tiles_y;
+      x0 = (tile % tiles_x) * kTileX;
+      n = tile / tiles_x;
+    } else {
+      x0 = (tile % tiles_x) * kTileX;
+      tile /= tiles_x;
+      y0 = (tile % tiles_y) * kTileY;
+      n = tile / tiles_y;
+    }
+  };
 
   uint4 ra[kAIters], rb[kBIters];
-  // global loads of chunk c (channels 32 c .. 32 c + 31) into ra, rb
-  auto fetch = [&](int c) {
+  // global loads of channels 32 c .. 32 c + 31 of the window and the weights
+  auto fetch_a = [&](int c) {
     const int cc = 32 * c;
 #pragma unroll
     for (int i = 0; i < kAIters; ++i) {
@@ -210,6 +342,8 @@ __device__ __forceinline__ void conv_lds_block(const ConvArgs& a, int tiles_x,
       }
       ra[i] = v;
     }
+  };
+  auto fetch_b = [&](int c) {
 #pragma unroll
     for (int i = 0; i < kBIters; ++i) {
       const int q = tid + 256 * i;
@@ -218,12 +352,12 @@ __device__ __forceinline__ void conv_lds_block(const ConvArgs& a, int tiles_x,
         const int tap = q / (kCO * 4), rem = q - tap * (kCO * 4);
         const int co = rem >> 2, g = rem & 3;
         v = *reinterpret_cast<const uint4*>(
-            a.w + (size_t)(co0 + co) * kpad + tap * cin + cc + 8 * g);
+            a.w + (size_t)(co0 + co) * kpad + tap * cin + 32 * c + 8 * g);
       }
       rb[i] = v;
     }
   };
-  auto stage = [&]() {
+  auto stage_a = [&]() {
 #pragma unroll
     for (int i = 0; i < kAIters; ++i) {
       const int q = tid + 256 * i;
@@ -233,6 +367,8 @@ __device__ __forceinline__ void conv_lds_block(const ConvArgs& a, int tiles_x,
         sA[(r * kWinX + xt) * 4 + lds_slot(g, xt)] = ra[i];
       }
     }
+  };
+  auto stage_b = [&]() {
 #pragma unroll
     for (int i = 0; i < kBIters; ++i) {
       const int q = tid + 256 * i;
@@ -245,16 +381,14 @@ __device__ __forceinline__ void conv_lds_block(const ConvArgs& a, int tiles_x,
   };
 
   f32x4 acc[4][kNT];
+  auto clear = [&]() {
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  fetch(0);
-  for (int c = 0; c < nchunks; ++c) {
-    __syncthreads();  // every wavefront is done reading the previous chunk
-    stage();
-    __syncthreads();
-    if (c + 1 < nchunks) fetch(c + 1);
+      for (int nt = 0; nt < kNT; ++nt)
+        acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto multiply = [&]() {
 #pragma unroll
     for (int tap = 0; tap < 9; ++tap) {
       const int dy = tap / 3, dx = tap % 3;  // window offsets 0..2
@@ -276,76 +410,125 @@ __device__ __forceinline__ void conv_lds_block(const ConvArgs& a, int tiles_x,
 #pragma unroll
         for (int nt = 0; nt < kNT; ++nt)
           acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              A[mt], B[nt], acc[mt][nt], 0, 0, 0);
+              B[nt], A[mt], acc[mt][nt], 0, 0, 0);
     }
-  }
-  const int y = y0 + wave;
-  if (y >= a.H) return;
+  };
+  f32x4 bias[kNT];
+  auto load_bias = [&]() {
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+    for (int nt = 0; nt < kNT; ++nt)
+      bias[nt] = conv_bias4(a, co0 + nt * 16 + 4 * grp);
+  };
+  auto store = [&](int sn, int sx, int sy) {
+    const int y = sy + wave;
+    if (y >= a.H) return;
 #pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) {
-      const int co = co0 + nt * 16 + row;
-      if (co >= a.cout) continue;
-      const float b = a.bias ? a.bias[co] : 0.0f;
+    for (int mt = 0; mt < 4; ++mt) {
+      const int x = sx + mt * 16 + row;
+      if (x >= a.W) continue;
+      const size_t p = ((size_t)sn * a.H + y) * a.W + x;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int x = x0 + mt * 16 + 4 * grp + j;
-        if (x >= a.W) continue;
-        const size_t p = ((size_t)n * a.H + y) * a.W + x;
-        float v = acc[mt][nt][j] + b;
-        if (a.relu) v = fmaxf(v, 0.0f);
-        if (a.yf)
-          a.yf[p * a.ys + co] = v;
-        else
-          a.y[p * a.ys + co] = (bf16)v;
+      for (int nt = 0; nt < kNT; ++nt)
+        conv_store4(a, p, co0 + nt * 16 + 4 * grp, acc[mt][nt], bias[nt],
+                    vec);
+    }
+  };
+
+  place(t);
+  fetch_a(0);
+  fetch_b(0);
+  if (kWalk) {
+    load_bias();
+    stage_b();
+    for (; t < t_end; ++t) {
+      __syncthreads();  // every wavefront is done reading the last window
+      stage_a();
+      __syncthreads();
+      const int sn = n, sx = x0, sy = y0;
+      if (t + 1 < t_end) {
+        place(t + 1);
+        fetch_a(0);
       }
+      clear();
+      multiply();
+      store(sn, sx, sy);
     }
-}
-
-// 32 output channels per work-group.  With one input chunk (32 input
-// channels) nothing overlaps a work-group's fetch, so that form is built
-// for three wavefronts per SIMD (168 VGPRs, a few spilled); with more
-// chunks the spills cost more than the extra wavefront gains and the
-// unconstrained build (two per SIMD) is used.  At 720p: the single-chunk
-// layers 143 -> 115 us, the others 3-12 % slower at three.  The
-// 64-channel form cannot reach three and keeps two.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
-k_conv_lds32_1chunk(ConvArgs a, int tiles_x, int tiles_y) {
-  conv_lds_block<2>(a, tiles_x, tiles_y);
-}
-
-__global__ void __launch_bounds__(256)
-k_conv_lds32(ConvArgs a, int tiles_x, int tiles_y) {
-  conv_lds_block<2>(a, tiles_x, tiles_y);
-}
-
-__global__ void __launch_bounds__(256)
-k_conv_lds64(ConvArgs a, int tiles_x, int tiles_y) {
-  conv_lds_block<4>(a, tiles_x, tiles_y);
-}
-
-hipError_t launch_conv(hipStream_t st, const ConvArgs& a) {
-  const long npix = (long)a.N * a.H * a.W;
-  const int cpad = conv_cpad(a.cout);
-  if (a.dil == 1 && a.c1 % 32 == 0 && a.c2 % 32 == 0 && a.c1 + a.c2 > 0) {
-    const int tiles_x = (a.W + kTileX - 1) / kTileX;
-    const int tiles_y = (a.H + kTileY - 1) / kTileY;
-    const unsigned g = (unsigned)((long)tiles_x * tiles_y * a.N);
-    if (cpad % 64 == 0)
-      NET_LAUNCH(k_conv_lds64, dim3(g, (unsigned)(cpad / 64)), dim3(256), 0,
-                 st, a, tiles_x, tiles_y);
-    if (a.c1 + a.c2 == 32)
-      NET_LAUNCH(k_conv_lds32_1chunk, dim3(g, (unsigned)(cpad / 32)),
-                 dim3(256), 0, st, a, tiles_x, tiles_y);
-    NET_LAUNCH(k_conv_lds32, dim3(g, (unsigned)(cpad / 32)), dim3(256), 0,
-               st, a, tiles_x, tiles_y);
+  } else {
+    clear();
+    for (int c = 0; c < nchunks; ++c) {
+      __syncthreads();  // every wavefront is done reading the previous chunk
+      stage_a();
+      stage_b();
+      __syncthreads();
+      if (c + 1 < nchunks) {
+        fetch_a(c + 1);
+        fetch_b(c + 1);
+      }
+      multiply();
+    }
+    load_bias();
+    store(n, x0, y0);
   }
-  const unsigned gx = (unsigned)((npix + kConvPix - 1) / kConvPix);
-  if (cpad % 64 == 0)
-    NET_LAUNCH(k_conv<4>, dim3(gx, (unsigned)(cpad / 64)), dim3(64), 0, st,
-               a);
-  NET_LAUNCH(k_conv<2>, dim3(gx, (unsigned)(cpad / 32)), dim3(64), 0, st, a);
+}
+
+// three wavefronts per SIMD
+template <int kNT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+k_conv_lds_walk(ConvArgs a, int tiles_x, int tiles_y, int tiles, bool vec) {
+  conv_lds_block<kNT, true>(a, tiles_x, tiles_y, tiles, vec);
+}
+
+// Two work-groups per CU, which the 64-channel form needs said: at 264
+// registers it ran one (64 -> 64 at 640 x 360: 49 us, 37 at 250 registers).
+template <int kNT>
+__global__ void __launch_bounds__(256, 2)
+k_conv_lds(ConvArgs a, int tiles_x, int tiles_y, int tiles, bool vec) {
+  conv_lds_block<kNT, false>(a, tiles_x, tiles_y, tiles, vec);
+}
+
+template <int kNT>
+static hipError_t launch_lds(hipStream_t st, const ConvArgs& a, bool vec) {
+  const int tiles_x = (a.W + kTileX - 1) / kTileX;
+  const int tiles_y = (a.H + kTileY - 1) / kTileY;
+  const int tiles = (int)((long)tiles_x * tiles_y * a.N);
+  NET_LAUNCH(k_conv_lds<kNT>,
+             dim3((unsigned)tiles, (unsigned)(conv_cpad(a.cout) / (16 * kNT))),
+             dim3(256), 0, st, a, tiles_x, tiles_y, tiles, vec);
+}
+
+template <int kNT>
+static hipError_t launch_walk(hipStream_t st, const ConvArgs& a, bool vec) {
+  const int tiles_x = (a.W + kTileX - 1) / kTileX;
+  const int tiles_y = (a.H + kTileY - 1) / kTileY;
+  const int tiles = (int)((long)tiles_x * tiles_y * a.N);
+  // work-groups that run at once (3 per CU), each a run of tiles
+  NET_LAUNCH(k_conv_lds_walk<kNT>,
+             dim3((unsigned)std::min(tiles, 768),
+                  (unsigned)((a.cout + 16 * kNT - 1) / (16 * kNT))),
+             dim3(256), 0, st, a, tiles_x, tiles_y, tiles, vec);
+}
+
+// All forms sum K in the order that their layers always had, so a layer
+// gives the same bits whichever runs.
+hipError_t launch_conv(hipStream_t st, const ConvArgs& a) {
+  const int cpad = conv_cpad(a.cout), cin = a.c1 + a.c2;
+  const bool vec = conv_vec_store(a);
+  if (a.dil == 1 && a.c1 % 32 == 0 && a.c2 % 32 == 0 && cin > 0) {
+    if (cin == 32)
+      return a.cout <= 16 ? launch_walk<1>(st, a, vec)
+                          : launch_walk<2>(st, a, vec);
+    return cpad % 64 == 0 ? launch_lds<4>(st, a, vec)
+                          : launch_lds<2>(st, a, vec);
+  }
+  // Tiles of 16 x 8 share the weights' loads among twice the pixels, but need
+  // enough wavefronts to hide them: 128 -> 128, dilation 2, at 160 x 90 (960
+  // wavefronts) takes 18 us with 16 x 8 and 17 with 16 x 4, dilation 4 and 8 18
+  // and 20 against 21; at 40 x 30 (128 wavefronts) 14-16 against 11.
+  const long waves = (long)((a.W + kLatX * a.dil - 1) / (kLatX * a.dil)) *
+                     ((a.H + 8 * a.dil - 1) / (8 * a.dil)) * a.dil * a.dil *
+                     a.N * (cpad / 16);
+  return waves >= 512 ? launch_lattice<8, 1, 4, 8>(st, a, vec)
+                      : launch_lattice<4, 1, 8, 4>(st, a, vec);
 }
 
 // ---------------------------------------------------------------------
