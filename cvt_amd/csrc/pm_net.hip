@@ -57,10 +57,18 @@ __device__ __forceinline__ void conv_store4(const ConvArgs& a, size_t p,
     v[j] = acc[j] + bias[j];
     if (a.relu) v[j] = fmaxf(v[j], 0.0f);
   }
+  float* yf = a.yf + p * a.ys + co;
+  if (a.yf2 && co >= a.split)
+    yf = a.yf2 + p * (a.cout - a.split) + (co - a.split);
   if (vec) {
+    if (a.mask) {
+      const bf16x4 m =
+          *reinterpret_cast<const bf16x4*>(a.mask + p * a.ys + co);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = (float)m[j] > 0.0f ? v[j] : 0.0f;
+    }
     if (a.yf) {
-      *reinterpret_cast<float4*>(a.yf + p * a.ys + co) =
-          make_float4(v[0], v[1], v[2], v[3]);
+      *reinterpret_cast<float4*>(yf) = make_float4(v[0], v[1], v[2], v[3]);
     } else {
       bf16x4 o;
 #pragma unroll
@@ -72,18 +80,20 @@ __device__ __forceinline__ void conv_store4(const ConvArgs& a, size_t p,
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     if (co + j >= a.cout) continue;
+    if (a.mask && !((float)a.mask[p * a.ys + co + j] > 0.0f)) v[j] = 0.0f;
     if (a.yf)
-      a.yf[p * a.ys + co + j] = v[j];
+      yf[j] = v[j];
     else
       a.y[p * a.ys + co + j] = (bf16)v[j];
   }
 }
 
 static bool conv_vec_store(const ConvArgs& a) {
-  const uintptr_t mask = a.yf ? 15 : 7;
-  const uintptr_t ptr = reinterpret_cast<uintptr_t>(
-      a.yf ? static_cast<const void*>(a.yf) : static_cast<const void*>(a.y));
-  return a.ys % 4 == 0 && a.cout % 4 == 0 && (ptr & mask) == 0;
+  const uintptr_t ptr = a.yf ? reinterpret_cast<uintptr_t>(a.yf) |
+                                   reinterpret_cast<uintptr_t>(a.yf2)
+                             : 2 * (reinterpret_cast<uintptr_t>(a.y) |
+                                    reinterpret_cast<uintptr_t>(a.mask));
+  return a.ys % 4 == 0 && a.cout % 4 == 0 && ptr % 16 == 0;
 }
 
 // ---------------------------------------------------------------------
@@ -788,74 +798,76 @@ hipError_t launch_flip_weights(hipStream_t st, const bf16* w, int cin,
              st, w, cin, cout, wt);
 }
 
-__global__ void __launch_bounds__(256)
-k_grad_mask(size_t n, const float* __restrict__ g, const bf16* __restrict__ y,
-            int relu, bf16* __restrict__ out) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  float v = g[i];
-  if (relu && !((float)y[i] > 0.0f)) v = 0.0f;
-  out[i] = (bf16)v;
+__device__ __forceinline__ void store_masked4(const float (&v)[4],
+                                              const bf16* y, bf16* out) {
+  const bf16x4 m = *reinterpret_cast<const bf16x4*>(y);
+  bf16x4 o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    o[j] = (bf16)((float)m[j] > 0.0f ? v[j] : 0.0f);
+  *reinterpret_cast<bf16x4*>(out) = o;
 }
 
-hipError_t launch_grad_mask(hipStream_t st, size_t n, const float* g,
-                            const bf16* y, int relu, bf16* out) {
-  NET_LAUNCH(k_grad_mask, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-             n, g, y, relu, out);
+// a thread: 4 consecutive channels of a pixel
+__global__ void __launch_bounds__(256)
+k_mask_pool(int N, int H, int W, int C, const float* __restrict__ g,
+            const float* __restrict__ gp, const bf16* __restrict__ y,
+            bf16* __restrict__ out) {
+  const unsigned C4 = C / 4;
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (size_t)N * H * W * C4) return;
+  const unsigned c = (unsigned)(i % C4) * 4;
+  const size_t q = i / C4;
+  const unsigned x = (unsigned)(q % W);
+  const size_t r = q / W;
+  const unsigned yy = (unsigned)(r % H), n = (unsigned)(r / H);
+  const float4 a = *reinterpret_cast<const float4*>(g + q * C + c);
+  const float4 b = *reinterpret_cast<const float4*>(
+      gp + (((size_t)n * (H / 2) + (yy >> 1)) * (W / 2) + (x >> 1)) * C + c);
+  const float v[4] = {a.x + 0.25f * b.x, a.y + 0.25f * b.y,
+                      a.z + 0.25f * b.z, a.w + 0.25f * b.w};
+  store_masked4(v, y + q * C + c, out + q * C + c);
+}
+
+hipError_t launch_mask_pool(hipStream_t st, int N, int H, int W, int C,
+                            const float* g, const float* gp, const bf16* y,
+                            bf16* out) {
+  if (C % 4) return hipErrorInvalidValue;
+  const size_t n = (size_t)N * H * W * (C / 4);
+  NET_LAUNCH(k_mask_pool, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
+             N, H, W, C, g, gp, y, out);
 }
 
 __global__ void __launch_bounds__(256)
-k_route_first(size_t npix, int c1, int c2, const float* __restrict__ t,
-              float* __restrict__ g1) {
+k_mask_up(int N, int H, int W, int C, const float* __restrict__ g,
+          const bf16* __restrict__ y, bf16* __restrict__ out) {
+  const unsigned C4 = C / 4;
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= npix * c1) return;
-  const size_t p = i / c1, c = i % c1;
-  g1[i] += t[p * (c1 + c2) + c];
-}
-
-__global__ void __launch_bounds__(256)
-k_route_second(int N, int H, int W, int c1, int c2, int up2,
-               const float* __restrict__ t, float* __restrict__ g2) {
-  const int H2 = up2 ? (H + 1) >> 1 : H, W2 = up2 ? (W + 1) >> 1 : W;
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (size_t)N * H2 * W2 * c2) return;
-  const int c = (int)(i % c2);
-  const size_t q = i / c2;
-  const int x2 = (int)(q % W2);
-  const size_t r = q / W2;
-  const int y2 = (int)(r % H2), n = (int)(r / H2);
-  const int ct = c1 + c2;
-  float s = 0.0f;
-  if (up2) {
-    for (int dy = 0; dy < 2; ++dy)
-      for (int dx = 0; dx < 2; ++dx) {
-        const int y = 2 * y2 + dy, x = 2 * x2 + dx;
-        if (y < H && x < W)
-          s += t[(((size_t)n * H + y) * W + x) * ct + c1 + c];
-      }
-  } else {
-    s = t[(((size_t)n * H + y2) * W + x2) * ct + c1 + c];
+  if (i >= (size_t)N * H * W * C4) return;
+  const unsigned c = (unsigned)(i % C4) * 4;
+  const size_t q = i / C4;
+  const unsigned x = (unsigned)(q % W);
+  const size_t r = q / W;  // image * H + row
+  const float* p = g + (2 * r * 2 * W + 2 * x) * C + c;
+  float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float4 t = *reinterpret_cast<const float4*>(
+        p + ((size_t)(k >> 1) * 2 * W + (k & 1)) * C);
+    v[0] += t.x;
+    v[1] += t.y;
+    v[2] += t.z;
+    v[3] += t.w;
   }
-  g2[i] += s;
+  store_masked4(v, y + q * C + c, out + q * C + c);
 }
 
-hipError_t launch_route_grad(hipStream_t st, int N, int H, int W, int c1,
-                             int c2, int up2, const float* t, float* g1,
-                             float* g2) {
-  const size_t npix = (size_t)N * H * W;
-  if (g1 && c1 > 0) {
-    (void)hipGetLastError();
-    hipLaunchKernelGGL(k_route_first,
-                       dim3((unsigned)((npix * c1 + 255) / 256)), dim3(256),
-                       0, st, npix, c1, c2, t, g1);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  if (!g2 || c2 == 0) return hipSuccess;
-  const size_t H2 = up2 ? (H + 1) / 2 : H, W2 = up2 ? (W + 1) / 2 : W;
-  const size_t n2 = (size_t)N * H2 * W2 * c2;
-  NET_LAUNCH(k_route_second, dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0,
-             st, N, H, W, c1, c2, up2, t, g2);
+hipError_t launch_mask_up(hipStream_t st, int N, int H, int W, int C,
+                          const float* g, const bf16* y, bf16* out) {
+  if (C % 4) return hipErrorInvalidValue;
+  const size_t n = (size_t)N * H * W * (C / 4);
+  NET_LAUNCH(k_mask_up, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
+             N, H, W, C, g, y, out);
 }
 
 __global__ void __launch_bounds__(256)
@@ -893,48 +905,29 @@ hipError_t launch_avgpool(hipStream_t st, int N, int H, int W, int C,
 }
 
 __global__ void __launch_bounds__(256)
-k_avgpool_grad(int N, int H, int W, int C, const float* __restrict__ gout,
-               float* __restrict__ gin) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (size_t)N * H * W * C) return;
-  const int c = (int)(i % C);
-  const size_t q = i / C;
-  const int x = (int)(q % W);
-  const size_t r = q / W;
-  const int y = (int)(r % H), n = (int)(r / H);
-  const int Ho = H / 2, Wo = W / 2;
-  gin[i] += 0.25f * gout[(((size_t)n * Ho + (y >> 1)) * Wo + (x >> 1)) * C + c];
-}
-
-hipError_t launch_avgpool_grad(hipStream_t st, int N, int H, int W, int C,
-                               const float* gout, float* gin) {
-  const size_t n = (size_t)N * H * W * C;
-  NET_LAUNCH(k_avgpool_grad, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-             st, N, H, W, C, gout, gin);
-}
-
-__global__ void __launch_bounds__(256)
 k_l1_loss(size_t npix, const float* __restrict__ o, int os,
           const float4* __restrict__ t, float wd, float wn, float inv_count,
-          float* __restrict__ g, float* __restrict__ loss) {
+          bf16* __restrict__ g, float* __restrict__ loss) {
   __shared__ float part[256];
   const size_t p = (size_t)blockIdx.x * 256 + threadIdx.x;
   float l = 0.0f;
   if (p < npix) {
     const float4 tv = t[p];
     const float* op = o + p * os;
-    float* gp = g + p * os;
-    for (int c = 0; c < os; ++c) gp[c] = 0.0f;
+    bf16x8 gp = zero8();
     if (tv.x >= 0.0f) {
       const float d[4] = {op[0] - tv.x, op[1] - tv.y, op[2] - tv.z,
                           op[3] - tv.w};
       const float w[4] = {wd, wn, wn, wn};
       for (int c = 0; c < 4; ++c) {
         l += w[c] * fabsf(d[c]);
-        gp[c] = d[c] > 0.0f ? w[c] * inv_count
-                            : (d[c] < 0.0f ? -w[c] * inv_count : 0.0f);
+        gp[c] = (bf16)(d[c] > 0.0f ? w[c] * inv_count
+                                   : (d[c] < 0.0f ? -w[c] * inv_count : 0.0f));
       }
     }
+    for (int c = 8; c < os; c += 8)
+      *reinterpret_cast<bf16x8*>(g + p * os + c) = zero8();
+    *reinterpret_cast<bf16x8*>(g + p * os) = gp;
   }
   part[threadIdx.x] = l;
   __syncthreads();
@@ -947,7 +940,8 @@ k_l1_loss(size_t npix, const float* __restrict__ o, int os,
 
 hipError_t launch_l1_loss(hipStream_t st, size_t npix, const float* o, int os,
                           const float* t, float wd, float wn, float inv_count,
-                          float* g, float* loss) {
+                          bf16* g, float* loss) {
+  if (os % 8) return hipErrorInvalidValue;
   NET_LAUNCH(k_l1_loss, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0,
              st, npix, o, os, reinterpret_cast<const float4*>(t), wd, wn,
              inv_count, g, loss);

@@ -32,7 +32,10 @@ __host__ __device__ inline int conv_cpad(int cout) {
 // w[co][k], co < conv_cpad(cout), k = tap * (c1 + c2) + ci < conv_kpad(c1 +
 // c2), tap = 3 (dy + 1) + (dx + 1), bf16, zero beyond the real ones.
 // Output (N x H x W, channel stride ys >= cout) with the bias (when not
-// null) and an optional ReLU: bf16 into y, or fp32 into yf when set.
+// null) and an optional ReLU: bf16 into y, or fp32 into yf when set.  For
+// the gradient of an input: mask (N x H x W, channel stride ys): the output
+// is 0 where it is not above 0; yf2: output channels from split on go there,
+// with channel stride cout - split.  split is a multiple of 4.
 struct ConvArgs {
   const bf16* x1 = nullptr;
   const bf16* x2 = nullptr;
@@ -44,6 +47,9 @@ struct ConvArgs {
   bf16* y = nullptr;
   float* yf = nullptr;
   int ys = 0;
+  const bf16* mask = nullptr;
+  float* yf2 = nullptr;
+  int split = 0;
 };
 hipError_t launch_conv(hipStream_t st, const ConvArgs& a);
 
@@ -59,31 +65,29 @@ hipError_t launch_conv_wgrad(hipStream_t st, const ConvArgs& a,
 hipError_t launch_flip_weights(hipStream_t st, const bf16* w, int cin,
                                int cout, bf16* wt);
 
-// g_bf16[i] = g[i] * (y[i] > 0) (ReLU) or g[i] (relu = 0), n elements
-hipError_t launch_grad_mask(hipStream_t st, size_t n, const float* g,
-                            const bf16* y, int relu, bf16* out);
-
-// t holds the input gradient of a concatenated input (N x H x W x (c1 +
-// c2), fp32): g1 += its first c1 channels; g2 += the other c2, summed over
-// 2 x 2 blocks when x2 was upsampled (up2).  g2 may be null (no gradient).
-hipError_t launch_route_grad(hipStream_t st, int N, int H, int W, int c1,
-                             int c2, int up2, const float* t, float* g1,
-                             float* g2);
+// Masked gradients, bf16, C a multiple of 4.  k_mask_pool: of a tensor whose
+// gradient is g (N x H x W x C, fp32) plus a quarter of that of its 2 x 2
+// average, gp; k_mask_up: of a tensor (N x H x W x C) read nearest-upsampled,
+// the sum of g (N x 2H x 2W x C) over 2 x 2 blocks.  0 where y is not above 0.
+hipError_t launch_mask_pool(hipStream_t st, int N, int H, int W, int C,
+                            const float* g, const float* gp, const bf16* y,
+                            bf16* out);
+hipError_t launch_mask_up(hipStream_t st, int N, int H, int W, int C,
+                          const float* g, const bf16* y, bf16* out);
 
 // 2 x 2 average pooling, bf16 (N x H x W x C -> N x H/2 x W/2 x C, H and
-// W even, C a multiple of 8), and its gradient: gin += 0.25 gout
+// W even, C a multiple of 8)
 hipError_t launch_avgpool(hipStream_t st, int N, int H, int W, int C,
                           const bf16* x, bf16* y);
-hipError_t launch_avgpool_grad(hipStream_t st, int N, int H, int W, int C,
-                               const float* gout, float* gin);
 
 // Masked L1 loss of the head output o (N x H x W x os fp32, channels 0..3
 // = disparity / kDispScale, nx, ny, nz) against t (N x H x W x 4; a
 // disparity below 0 marks a pixel without a target): g = dloss / do
-// (channels 0..3, 0 elsewhere), loss += sum / count.  count: valid pixels.
+// (channels 0..3, 0 elsewhere; bf16, os a multiple of 8), loss += sum /
+// count.  count: valid pixels.
 hipError_t launch_l1_loss(hipStream_t st, size_t npix, const float* o,
                           int os, const float* t, float wd, float wn,
-                          float inv_count, float* g, float* loss);
+                          float inv_count, bf16* g, float* loss);
 
 // Adam on n fp32 parameters; writes their bf16 copy
 hipError_t launch_adam(hipStream_t st, size_t n, float* w, const float* g,
