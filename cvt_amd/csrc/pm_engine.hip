@@ -179,6 +179,7 @@ struct Lane {
   const float* __restrict__ col12;  // other view's packed colour (0, 0)
   float flo, fhi;       // x' in [flo, fhi] reads inside image and window
   float safe;           // a column that does: the block's first
+  int sub;              // this lane's number in its pixel's team
 };
 
 // Block prologue shared by the cost-evaluating kernels, for the block
@@ -190,13 +191,16 @@ struct Lane {
 // color) & 1) of its row, the pixel of the pass's colour.  Must be reached
 // by every thread of the block; the block is 64 kWX x kRows threads, and
 // lanes of rows from row_end on are invalid.
-template <bool kGrad, bool kRB, int kRows, int kWX = 1, bool kWin = false>
+// kTeam lanes share a pixel (see "Teams"), so the block covers kTeam times
+// fewer columns.
+template <bool kGrad, bool kRB, int kRows, int kWX = 1, bool kWin = false,
+          int kTeam = 1>
 __device__ Lane block_setup_at(const Geometry& g, const ViewBufs& self,
                                const ViewBufs& other, float4* smem, int x0,
                                int y0, int row_end, Window win = Window()) {
   const int R = g.R, W = g.W, H = g.H;
   constexpr int kThreads = kTX * kWX * kRows;
-  const int cols = kRB ? 2 * kTX * kWX : kTX * kWX;
+  const int cols = (kRB ? 2 : 1) * kTX * kWX / kTeam;
   const int TW = cols + 2 * R, TH = kRows + 2 * R;
   const int tid = threadIdx.y * (kTX * kWX) + threadIdx.x;
   const size_t gplane = (size_t)g.TS * H;
@@ -235,8 +239,8 @@ __device__ Lane block_setup_at(const Geometry& g, const ViewBufs& self,
   const int wx0 =
       x0 + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTX) *
                (kRB ? 2 * kTX : kTX);
-  const int lx = kRB ? 2 * (int)threadIdx.x + ((y0 + ly + g.color) & 1)
-                     : (int)threadIdx.x;
+  const int lx0 = (int)threadIdx.x / kTeam;
+  const int lx = kRB ? 2 * lx0 + ((y0 + ly + g.color) & 1) : lx0;
   Lane L;
   L.W = W;
   L.H = H;
@@ -258,10 +262,12 @@ __device__ Lane block_setup_at(const Geometry& g, const ViewBufs& self,
   L.tex2 = other.tex + kTexPadL;
   L.tame = false;
   L.edge = true;
-  if (kWin) {
+  L.sub = (int)threadIdx.x % kTeam;
+  if (kWin || kTeam > 1)
     L.tame = __builtin_amdgcn_readfirstlane(
                  (int)(*wild_word(self.tex, g.TS, H) |
                        *wild_word(other.tex, g.TS, H))) == 0;
+  if (kWin) {
     L.edge = wx0 - R < 1 || wx0 + (kRB ? 2 * kTX : kTX) - 1 + R > W - 2;
     L.wcols = win.cols;
     L.wstride = win.cols + kWinEdge;
@@ -972,12 +978,132 @@ __device__ float cost_eval_cg(const Lane& L, float4 s, bool active,
   return ret / wsum;
 }
 
+// ---------------------------------------------------------------------
+// Teams.  A small image has fewer pixels than the GPU needs lanes: 320 x 240
+// is 1200 wavefronts for 1024 SIMDs, and a wavefront alone on its SIMD waits
+// for every load and for every instruction before the next.  There four lanes
+// (a quad) share a pixel: each takes every fourth tap of a patch row and
+// forms the tap's terms, then all four add the quad's terms up in the order
+// of the taps, each lane's broadcast by DPP, so that every lane holds the
+// sums and the bits are those of one lane's.  A tap that does not count has
+// terms of -0, which leave any sum as it is.
+// Three iterations of 320 x 240, R = 5: 4.85 -> 3.01 ms; 451 x 333, R = 7,
+// red-black: 17.8 -> 12.4.  Tried on top: the wide tile's window of gradients
+// in LDS (3.12; 16.9, for the work-groups it keeps off a CU), one image row
+// per work-group (no difference), all nine KLT sums in every lane (3.17;
+// 13.0).
+// ---------------------------------------------------------------------
+constexpr int kTeamLanes = 4;
+
+template <int kLane>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v),
+                                                 0x55 * kLane, 0xf, 0xf, true));
+}
+
+// add(term a, term b, tap of the quad) for the quad's four taps in order
+template <typename Add>
+__device__ __forceinline__ void quad_sum(float a, float b, Add add) {
+  add(quad_lane<0>(a), quad_lane<0>(b), 0);
+  add(quad_lane<1>(a), quad_lane<1>(b), 1);
+  add(quad_lane<2>(a), quad_lane<2>(b), 2);
+  add(quad_lane<3>(a), quad_lane<3>(b), 3);
+}
+
+// cost_eval and cost_eval_cg by a team; kTame: see "Tame images"
+template <int kKind, bool kTame>
+__device__ __forceinline__ float cost_team(const Lane& L, float4 s,
+                                           float mincost, bool active,
+                                           float* quot) {
+  constexpr bool kGrad = kKind == kCostColorGrad;
+  const int R = L.R, W = L.W;
+  bool live = active && L.valid;
+  float res = 0.0f;
+  if (!kGrad && live) {
+    const float xp = transform(s, L.xf, L.yf);
+    if (!(finite_f(s.x) && finite_f(s.y) && finite_f(s.z)) ||
+        to_normal(s).z < kNormalZMin || xp < 0.0f || xp >= L.Wf) {
+      res = 1e5f;
+      live = false;
+    }
+  }
+  const float cw = kGrad ? L.kw : L.cw;
+  const float negw = vconst(-cw), twenty = vconst(20.0f);
+  float sum = 0.0f, wsum = 0.0f;
+  for (int dy = -R; dy <= R; ++dy) {
+    if (!__any(live)) break;
+    const int qy = L.y + dy;  // uniform
+    if (qy < 0 || qy >= L.H) continue;
+    if (!live) continue;
+    const float rowb = s.y * (float)qy;  // transform(), b y per row
+    const float4* __restrict__ srow = L.tex2 + (size_t)qy * L.TS;
+    const LdsRow trow = L.trow0 + (dy + R) * L.TW;
+    for (int i0 = 0; i0 <= 2 * R; i0 += kTeamLanes) {
+      const int i = i0 + L.sub, x = L.x + i - R;
+      const float xq = fmaf(s.x, (float)x, rowb) + s.z;
+      float w = -0.0f, C = 0.0f;
+      if (i <= 2 * R && x >= 0 && x < W && xq >= 0.0f && xq < L.Wf) {
+        const float4 t1 = lds_at(trow, i);
+        const float dr = t1.x - L.tc.x, dg = t1.y - L.tc.y,
+                    db = t1.z - L.tc.z;
+        w = kTame ? weight_tame(dr, dg, db, negw)
+                  : support_weight(dr, dg, db, cw);
+        const float fq = floorf(xq);
+        const float4* __restrict__ tq = srow + (int)fq;
+        const Sample s2 =
+            lerp_texels(texel_at(tq, L.GP), texel_at(tq + 1, L.GP), xq - fq);
+        if (kGrad) {
+          const float4 g1 = lds_at(trow, L.GT + i);
+          const float sc = (fminf(fabsf(t1.x - s2.r), 0.05f) +
+                            fminf(fabsf(t1.y - s2.g), 0.05f)) +
+                           fminf(fabsf(t1.z - s2.b), 0.05f);
+          const float sg = ((fminf(fabsf(g1.x - s2.grad.x), 0.05f) +
+                             fminf(fabsf(g1.y - s2.grad.y), 0.05f)) +
+                            fminf(fabsf(g1.z - s2.grad.z), 0.05f)) +
+                           fminf(fabsf(g1.w - s2.grad.w), 0.05f);
+          C = fmaf(0.05f, sc, (1.0f - 0.05f) * sg);
+        } else {
+          const uint32_t m1 = __float_as_uint(t1.w);
+          float c0, c1, c2, n;
+          if (kTame) {
+            c0 = clamp20(s2.r - t1.x, twenty);
+            c1 = clamp20(s2.g - t1.y, twenty);
+            c2 = clamp20(s2.b - t1.z, twenty);
+            n = sign_mismatches8f(m1, s2.grad);
+          } else {
+            c0 = fminf(fabsf(s2.r - t1.x), 0.05f) * 20.0f;
+            c1 = fminf(fabsf(s2.g - t1.y), 0.05f) * 20.0f;
+            c2 = fminf(fabsf(s2.b - t1.z), 0.05f) * 20.0f;
+            n = (float)sign_mismatches8(m1, s2.grad);
+          }
+          C = fmaf(0.02734375f, n, 0.125f * (0.33f * ((c0 + c1) + c2)));
+        }
+      }
+      quad_sum(w, C, [&](float wj, float Cj, int) {
+        sum = fmaf(wj, Cj, sum);
+        wsum += wj;
+      });
+    }
+    if (!kGrad && sum / L.bilw >= mincost) {
+      res = 1.0f;
+      live = false;
+    }
+  }
+  if (kGrad) return sum / wsum;
+  if (live) res = (wsum <= 1.0f) ? 1.1f : sum / wsum;
+  if (quot) *quot = sum / L.bilw;
+  return res;
+}
+
 // the candidate cost the kernels' patch_eval selects
-template <int kKind, bool kCount, bool kWin = false>
+template <int kKind, bool kCount, bool kWin = false, int kTeam = 1>
 __device__ __forceinline__ float cost_any(const Lane& L, float4 s,
                                           float mincost, bool active,
                                           uint32_t* ntaps,
                                           float* quot = nullptr) {
+  if (kTeam > 1)
+    return L.tame ? cost_team<kKind, true>(L, s, mincost, active, quot)
+                  : cost_team<kKind, false>(L, s, mincost, active, quot);
   // the counting pass takes the general loops, which count
   const bool tame = kWin && !kCount && L.tame;  // uniform
   if (kKind == kCostColorGrad)
@@ -1122,9 +1248,91 @@ __device__ float4 klt_solve(float4 s, const float (&J)[3],
   return mk4(s.x - r0, s.y - r1, s.z - r2, s.w - 1e5f);
 }
 
-template <bool kWin>
+// klt_pass_general by a team.  The nine sums are spread over the quad: each
+// lane keeps one of J, one of H00, H01, H02, H11 (A) and one of H12, H22 (B),
+// its coefficients chosen by the constants u, v (c = u px + v, exact for u 0
+// or 1).
+template <bool kTame>
+__device__ __forceinline__ float4 klt_team(const Lane& L, float4 s) {
+  const int R = L.R, W = L.W;
+  float J = 0.0f, A = 0.0f, B = 0.0f;
+  const float negw = vconst(-L.cw), twenty = vconst(20.0f);
+  const float ja = L.sub == 0 ? 1.0f : 0.0f;                // px | py | 1
+  const float aa = L.sub == 3 ? 0.0f : 1.0f;                // px px px py
+  const float ba = L.sub == 0 ? 1.0f : 0.0f;                // px py 1 py
+  if (L.valid) {
+    for (int dy = -R; dy <= R; ++dy) {
+      const int qy = L.y + dy;  // uniform
+      if (qy < 0 || qy >= L.H) continue;
+      const float py = (float)qy;
+      const float rowb = s.y * py;  // transform(), b y per row
+      const float4* __restrict__ srow = L.tex2 + (size_t)qy * L.TS;
+      const LdsRow trow = L.trow0 + (dy + R) * L.TW;
+        const float jb = L.sub == 0 ? 0.0f : (L.sub == 1 ? py : 1.0f);
+      const float ab = L.sub == 3 ? py : 0.0f;
+      const float bb = L.sub == 0 ? 0.0f : (L.sub == 2 ? 1.0f : py);
+      const float cB = L.sub == 0 ? py : 1.0f;              // py 1
+      for (int i0 = 0; i0 <= 2 * R; i0 += kTeamLanes) {
+        const int i = i0 + L.sub, x = L.x + i - R;
+        float gj = -0.0f, h = -0.0f;
+        if (i <= 2 * R && x >= 1 && x < W - 1) {
+          const float xq = fmaf(s.x, (float)x, rowb) + s.z;
+          const float xc = fmaxf(fminf(xq, L.Wf), -1.0f);
+          const float xp1 = xc + 1.0f;
+          const float fl = floorf(xc), flp = floorf(xp1);
+          const float a = xc - fl, ap = xp1 - flp;
+          const float4* __restrict__ tq = srow + (int)fl;
+          const Texel tw0 = texel_at(tq - 1, L.GP), tw1 = texel_at(tq, L.GP),
+                      tw2 = texel_at(tq + 1, L.GP),
+                      tw3 = texel_at(tq + 2, L.GP);
+          const Sample sm = lerp_texels(tw0, tw1, a);
+          const Sample s0 = lerp_texels(tw1, tw2, a);
+          Sample sp = lerp_texels(tw2, tw3, ap);
+          if (flp != fl + 1.0f)
+            sp = lerp_texels(tw3, texel_at(tq + 3, L.GP), ap);
+          const float4 t1 = lds_at(trow, i);
+          const float v0 = t1.x - L.tc.x, v1 = t1.y - L.tc.y,
+                      v2 = t1.z - L.tc.z;
+          const uint32_t ga = __float_as_uint(t1.w);
+          const float w1 = kTame ? weight_tame(v0, v1, v2, negw)
+                                 : support_weight(v0, v1, v2, L.cw);
+          auto term = [&](const Sample& t) {
+            if (kTame)
+              return klt_term_tame(Rgb{t.r, t.g, t.b}, t.grad, v0, v1, v2, ga,
+                                   w1 * (0.125f * 0.33f), w1 * 0.02734375f,
+                                   twenty);
+            return klt_term(t, v0, v1, v2, ga, (w1 * 0.125f) * 0.33f,
+                            w1 * 0.875f);
+          };
+          const float C = term(s0), Cxp = term(sp), Cxm = term(sm);
+          const float curv = fmaf(-2.0f, C, Cxp + Cxm);
+          if (curv > 0.0f) {
+            gj = (w1 * (Cxm - Cxp)) * 0.5f;
+            h = w1 * curv;
+          }
+        }
+        // a tap that counts has px >= 1; |px| keeps the others' terms -0
+        const float px0 = L.xf + (float)(i0 - R);
+        quad_sum(gj, h, [&](float g, float hj, int j) {
+          const float px = fabsf(px0 + (float)j);
+          J = fmaf(g, fmaf(px, ja, jb), J);
+          A = A + hj * (fmaf(px, aa, ab) * fmaf(px, ba, bb));
+          B = B + hj * cB;
+        });
+      }
+    }
+  }
+  const float Js[3] = {quad_lane<0>(J), quad_lane<1>(J), quad_lane<2>(J)};
+  const float Hs[6] = {quad_lane<0>(A), quad_lane<1>(A), quad_lane<2>(A),
+                       quad_lane<3>(A), quad_lane<0>(B), quad_lane<1>(B)};
+  return klt_solve(s, Js, Hs);
+}
+
+template <bool kWin, int kTeam>
 __device__ __forceinline__ float4 klt_pass(const Lane& L, float4 s,
                                            bool dead) {
+  if (kTeam > 1)
+    return L.tame ? klt_team<true>(L, s) : klt_team<false>(L, s);
   return kWin && L.tame ? klt_pass_tame(L, s, dead) : klt_pass_general(L, s);
 }
 
@@ -1445,12 +1653,14 @@ __device__ __forceinline__ void scatter(float4 self, int x, int y, int W,
 // (counters[1]) this block evaluates; the results are identical.
 // kRB: one pass of the red-black schedule (g.color); pass 1 reads the
 // neighbours of colour 0 from a.fresh, the planes pass 0 just wrote.
-template <int kKind, bool kCount, bool kRB, int kRows, int kWX, bool kWin>
+// kTeam: lanes per pixel, all of which hold its planes and costs.
+template <int kKind, bool kCount, bool kRB, int kRows, int kWX, bool kWin,
+          int kTeam = 1>
 __device__ __forceinline__ void propagate_block(
     const Geometry& g, const PropagateArgs& a, unsigned long long* counters,
     float4* smem, int x0, int y0, int row_end, Window win) {
   const Lane L =
-      block_setup_at<kKind == kCostColorGrad, kRB, kRows, kWX, kWin>(
+      block_setup_at<kKind == kCostColorGrad, kRB, kRows, kWX, kWin, kTeam>(
           g, a.self, a.other, smem, x0, y0, row_end, win);
   if (!__any(L.valid)) return;  // no barrier follows
   const int W = g.W, H = g.H;
@@ -1547,7 +1757,7 @@ __device__ __forceinline__ void propagate_block(
       for (int it = 0; it < kKltPasses; ++it) {
         const bool dead = sure && !finite_plane(cand);
         if (!__any(L.valid && !dead)) break;
-        cand = klt_pass<kWin>(L, cand, dead);
+        cand = klt_pass<kWin, kTeam>(L, cand, dead);
       }
     }
     // minimalCost (pmhstereo.cl:873-877).  With theta = 0 and no smooth
@@ -1572,8 +1782,8 @@ __device__ __forceinline__ void propagate_block(
     const bool flat = !kCount && k == kCandSmooth && a.flat_cost;
     float w = 0.0f, q = 0.0f;
     if (!(flat && a.flat_known))
-      w = cost_any<kKind, kCount, kWin>(L, cand, flat ? 1e10f : mincost,
-                                        active, nc, &q);
+      w = cost_any<kKind, kCount, kWin, kTeam>(
+          L, cand, flat ? 1e10f : mincost, active, nc, &q);
     if (flat && active) {
       float* fc = a.flat_cost + L.p * kFlatCosts;
       if (a.flat_known) {
@@ -1593,7 +1803,7 @@ __device__ __forceinline__ void propagate_block(
         self = cand;
     }
   }
-  if (!L.valid) return;
+  if (!L.valid || L.sub) return;
   if (a.viewout) scatter(self, L.x, L.y, W, a.lr, a.viewout);
   a.out[L.p] = self;
   if (kCount) {
@@ -1609,7 +1819,8 @@ __device__ __forceinline__ void propagate_block(
 }
 
 // The single-image launch: one tile block per work-group.
-template <int kKind, bool kCount, bool kRB, int kRows, int kWX, bool kWin>
+template <int kKind, bool kCount, bool kRB, int kRows, int kWX, bool kWin,
+          int kTeam>
 __global__ void __launch_bounds__(64 * kWX * kRows)
 __attribute__((amdgpu_waves_per_eu(4, 4)))
 k_propagate(Geometry g, PropagateArgs a, unsigned long long* counters,
@@ -1618,9 +1829,9 @@ k_propagate(Geometry g, PropagateArgs a, unsigned long long* counters,
   int bx, by;
   xcd_block(&bx, &by);
   const int row0 = g.band0 * kBandRows;
-  propagate_block<kKind, kCount, kRB, kRows, kWX, kWin>(
-      g, a, counters, smem, bx * (kRB ? 2 : 1) * kTX * kWX, row0 + by * kRows,
-      g.row_end(), win);
+  propagate_block<kKind, kCount, kRB, kRows, kWX, kWin, kTeam>(
+      g, a, counters, smem, bx * (kRB ? 2 : 1) * kTX * kWX / kTeam,
+      row0 + by * kRows, g.row_end(), win);
 }
 
 // view scatter alone, from a stored field: rebuilds the buffer the field's
@@ -1652,7 +1863,7 @@ k_klt_field(Geometry g, ViewBufs self, ViewBufs other,
   extern __shared__ float4 smem[];
   const Lane L = block_setup<false>(g, self, other, smem);
   float4 s = L.valid ? planes[L.p] : mk4(0.0f, 0.0f, 0.0f, 0.0f);
-  for (int i = 0; i < passes; ++i) s = klt_pass<false>(L, s, false);
+  for (int i = 0; i < passes; ++i) s = klt_pass<false, 1>(L, s, false);
   if (L.valid) out[L.p] = s;
 }
 
@@ -2156,19 +2367,20 @@ hipError_t launch_viewbuf_clear(hipStream_t st, const Geometry& g,
   PM_LAUNCH(k_viewbuf_clear, dim3(blocks), dim3(256), 0, st, g.npix, vbuf);
 }
 
-template <int kKind, bool kCount, bool kRB, int kRows, int kWX, bool kWin>
+template <int kKind, bool kCount, bool kRB, int kRows, int kWX, bool kWin,
+          int kTeam = 1>
 static hipError_t launch_propagate_tile(hipStream_t st, const Geometry& g,
                                         const PropagateArgs& a,
                                         unsigned long long* counters,
                                         size_t lds, Window win) {
-  const int cols = (kRB ? 2 : 1) * kTX * kWX;
+  const int cols = (kRB ? 2 : 1) * kTX * kWX / kTeam;
   const int rows = g.row_end() - g.band0 * kBandRows;
   const dim3 grid((unsigned)((g.W + cols - 1) / cols),
                   (unsigned)((rows + kRows - 1) / kRows));
   const hipError_t e =
-      allow_lds(k_propagate<kKind, kCount, kRB, kRows, kWX, kWin>, lds);
+      allow_lds(k_propagate<kKind, kCount, kRB, kRows, kWX, kWin, kTeam>, lds);
   if (e != hipSuccess) return e;
-  PM_LAUNCH((k_propagate<kKind, kCount, kRB, kRows, kWX, kWin>), grid,
+  PM_LAUNCH((k_propagate<kKind, kCount, kRB, kRows, kWX, kWin, kTeam>), grid,
             dim3(kTX * kWX, kRows), lds, st, g, a, counters, win);
 }
 
@@ -2197,6 +2409,25 @@ long long wide_tiles(int W, int H) {
          ((H + kWideRows - 1) / kWideRows);
 }
 
+// Teams pay while the image is too small to fill the GPU with one lane per
+// pixel.  The work of a team is its slots, 4 ceil((2 R + 1) / 4) a patch row,
+// so the line is on pixels times slots per tap; below R = 3 what all four
+// lanes do alike weighs more.  Time with teams against without, census,
+// Jacobi (red-black):
+//   R                1     2     3     4     5     6     7
+//   160 x 120            .67         .53   .45
+//   400 x 300     1.00  1.00   .78   .82   .69   .74   .66
+//                 (.82) (.81) (.61) (.65) (.53) (.55) (.47)
+//   512 x 384     1.25  1.21   .90   .95   .79   .85   .75
+//                (1.18)(1.17) (.88) (.94) (.79) (.85) (.75)
+//   560 x 416     1.43  1.41  1.06  1.13   .94  1.01   .90
+//                (1.21)(1.16) (.87) (.93) (.77) (.83) (.73)
+static bool team_pays(int R, int W, int H) {
+  const long long taps = 2 * R + 1;
+  const long long slots = (taps + kTeamLanes - 1) / kTeamLanes * kTeamLanes;
+  return (long long)W * H * slots <= taps * (R < 3 ? 150000 : 262144);
+}
+
 template <int kKind, bool kRB>
 static hipError_t launch_propagate_kind(hipStream_t st, const Geometry& g,
                                         const PropagateArgs& a,
@@ -2213,6 +2444,14 @@ static hipError_t launch_propagate_kind(hipStream_t st, const Geometry& g,
   if (counters)
     return launch_propagate_tile<kKind, true, kRB, kTY, 1, false>(
         st, g, a, counters, lds, Window());
+  // (a radius whose 64 x 4 tile does not fit is refused below)
+  if (lds <= kLdsPerCu && team_pays(g.R, g.W, g.H))
+    return launch_propagate_tile<kKind, false, kRB, kTY, 1, false, kTeamLanes>(
+        st, g, a, counters,
+        std::max(tile_lds_bytes(g.R, kKind, (kRB ? 2 : 1) * kTX / kTeamLanes,
+                                kTY, 0),
+                 lds_floor),
+        Window());
   return launch_propagate_tile<kKind, false, kRB, kTY, 1, false>(
       st, g, a, counters, lds, Window());
 }
