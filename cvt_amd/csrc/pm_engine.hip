@@ -1,17 +1,18 @@
 // pm_engine.hip -- gfx950 kernels of the PatchMatch stereo engine.
 //
 // Work decomposition (kernels that evaluate plane costs):
-//  - a work-group is a 64 x 4 pixel block, each wavefront one row of 64
-//    consecutive pixels; blocks are renumbered so that each XCD walks one
-//    contiguous band of the image (its L2 then holds the rows the band
-//    reads);
+//  - a work-group is a block of pixels, each wavefront a run of one row: 64
+//    x 4 pixels in general; for the propagate also 128 x 8 with a window of
+//    the other view (the wide tile, images that fill the GPU with it), or
+//    16 x 4 with four lanes per pixel (teams, images that do not fill it);
+//  - blocks are renumbered so that each XCD walks one contiguous band of
+//    the image (its L2 then holds the rows the band reads);
 //  - the block stages its own-view tile (pixels plus an r halo: colour and
 //    gradient sign bits) in LDS once; support weights are recomputed per
 //    tap from that tile instead of being streamed from HBM;
-//  - the other view is sampled straight from its colour and gradient
-//    planes (two adjacent 16-byte records of each per linear sample), so
-//    a wavefront's gather of one plane spans half the cache lines that
-//    interleaved 32-byte texels would.
+//  - the other view is sampled from its colour and gradient planes (two
+//    adjacent 16-byte records of each per linear sample), by the wide tile
+//    from packed 12-byte colours and the window's gradients in LDS.
 // The cost loops run wave-uniformly over patch rows (one image row per
 // wavefront) and every lane stays resident (no early return): lanes are
 // masked with flags, and kernels reach the block barrier with all threads.
