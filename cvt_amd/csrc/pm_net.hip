@@ -776,26 +776,38 @@ hipError_t launch_conv_wgrad(hipStream_t st, const ConvArgs& a, const bf16* g,
 // ---------------------------------------------------------------------
 // small kernels
 // ---------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
-k_flip_weights(const bf16* __restrict__ w, int cin, int cout,
-               bf16* __restrict__ wt) {
-  const int kpt = conv_kpad(cout), rows = conv_cpad(cin);
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (long)rows * kpt) return;
-  const int ci = (int)(i / kpt), kk = (int)(i % kpt);
+struct FlipTable {
+  FlipLayer l[kMaxFlips];
+};
+
+// a row of work-groups per layer: 16 launches of 4 us each were 0.1 ms of a
+// training step
+__global__ void __launch_bounds__(256) k_flip_weights(FlipTable t) {
+  const FlipLayer& f = t.l[blockIdx.y];
+  const int kpt = conv_kpad(f.cout), rows = conv_cpad(f.cin);
+  const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+  if (i >= rows * kpt) return;
+  const int ci = i / kpt, kk = i - ci * kpt;
   bf16 v = (bf16)0.0f;
-  if (ci < cin && kk < 9 * cout) {
-    const int t = kk / cout, co = kk - t * cout;
-    v = w[(size_t)co * conv_kpad(cin) + (size_t)(8 - t) * cin + ci];
+  if (ci < f.cin && kk < 9 * f.cout) {
+    const int tap = kk / f.cout, co = kk - tap * f.cout;
+    v = f.w[(size_t)co * conv_kpad(f.cin) + (size_t)(8 - tap) * f.cin + ci];
   }
-  wt[i] = v;
+  f.wt[i] = v;
 }
 
-hipError_t launch_flip_weights(hipStream_t st, const bf16* w, int cin,
-                               int cout, bf16* wt) {
-  const long n = (long)conv_cpad(cin) * conv_kpad(cout);
-  NET_LAUNCH(k_flip_weights, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-             st, w, cin, cout, wt);
+hipError_t launch_flip_weights(hipStream_t st, const FlipLayer* layers,
+                               int n) {
+  if (n < 1 || n > kMaxFlips) return hipErrorInvalidValue;
+  FlipTable t;
+  int most = 0;
+  for (int l = 0; l < n; ++l) {
+    t.l[l] = layers[l];
+    most = std::max(most, conv_cpad(layers[l].cin) *
+                              conv_kpad(layers[l].cout));
+  }
+  NET_LAUNCH(k_flip_weights, dim3((unsigned)((most + 255) / 256), (unsigned)n),
+             dim3(256), 0, st, t);
 }
 
 __device__ __forceinline__ void store_masked4(const float (&v)[4],
@@ -909,9 +921,9 @@ k_l1_loss(size_t npix, const float* __restrict__ o, int os,
           const float4* __restrict__ t, float wd, float wn, float inv_count,
           bf16* __restrict__ g, float* __restrict__ loss) {
   __shared__ float part[256];
-  const size_t p = (size_t)blockIdx.x * 256 + threadIdx.x;
   float l = 0.0f;
-  if (p < npix) {
+  for (size_t p = (size_t)blockIdx.x * 256 + threadIdx.x; p < npix;
+       p += (size_t)gridDim.x * 256) {
     const float4 tv = t[p];
     const float* op = o + p * os;
     bf16x8 gp = zero8();
@@ -942,7 +954,11 @@ hipError_t launch_l1_loss(hipStream_t st, size_t npix, const float* o, int os,
                           const float* t, float wd, float wn, float inv_count,
                           bf16* g, float* loss) {
   if (os % 8) return hipErrorInvalidValue;
-  NET_LAUNCH(k_l1_loss, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0,
+  // few work-groups, since each ends with an atomic add to the one sum
+  // (1.6 million pixels in 6144: 84 us)
+  NET_LAUNCH(k_l1_loss,
+             dim3((unsigned)std::min<size_t>((npix + 255) / 256, 1024)),
+             dim3(256), 0,
              st, npix, o, os, reinterpret_cast<const float4*>(t), wd, wn,
              inv_count, g, loss);
 }

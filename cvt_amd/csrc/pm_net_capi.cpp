@@ -246,10 +246,14 @@ int forward(pm_net* n, hipStream_t st, float* out = nullptr) {
 }
 
 int refresh_flipped(pm_net* n) {
-  for (int l = 1; l < kConvs; ++l)
-    NET_HIP(n, pm::net::launch_flip_weights(
-                   n->stream, as<bf16>(n->w16) + n->woff[l], conv_cin(l),
-                   conv_cout(l), as<bf16>(n->wflip[l])));
+  pm::net::FlipLayer f[kConvs - 1];
+  for (int l = 1; l < kConvs; ++l) {
+    f[l - 1].w = as<bf16>(n->w16) + n->woff[l];
+    f[l - 1].wt = as<bf16>(n->wflip[l]);
+    f[l - 1].cin = conv_cin(l);
+    f[l - 1].cout = conv_cout(l);
+  }
+  NET_HIP(n, pm::net::launch_flip_weights(n->stream, f, kConvs - 1));
   return PM_OK;
 }
 

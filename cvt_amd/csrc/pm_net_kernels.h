@@ -62,8 +62,15 @@ hipError_t launch_conv_wgrad(hipStream_t st, const ConvArgs& a,
 // w'[ci][k'] for the gradient of the input: the convolution of the output
 // gradient (cout channels) with the flipped, transposed kernel, k' = (8 -
 // tap) * cout + co; w' has conv_cpad(cin) rows of conv_kpad(cout)
-hipError_t launch_flip_weights(hipStream_t st, const bf16* w, int cin,
-                               int cout, bf16* wt);
+// for up to kMaxFlips layers in one launch
+struct FlipLayer {
+  const bf16* w = nullptr;
+  bf16* wt = nullptr;
+  int cin = 0, cout = 0;
+};
+constexpr int kMaxFlips = 16;
+hipError_t launch_flip_weights(hipStream_t st, const FlipLayer* layers,
+                               int n);
 
 // Masked gradients, bf16, C a multiple of 4.  k_mask_pool: of a tensor whose
 // gradient is g (N x H x W x C, fp32) plus a quarter of that of its 2 x 2
