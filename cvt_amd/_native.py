@@ -88,6 +88,8 @@ SIGNATURES = {
     "pm_net_set_params": (_i, [_p, _p, ctypes.c_size_t]),
     "pm_net_get_grads": (_i, [_p, _p, ctypes.c_size_t]),
     "pm_net_forward": (_i, [_p, _p, _i, _i, _i, _p]),
+    "pm_net_conv_selftest": (_i, [_p, _p, _i, _p, _i, _i, _i, _i, _i, _i, _i,
+                                  _p, _p, _p, _p, _p]),
     "pm_net_train_step": (_i, [_p, _p, _p, _i, _i, _i, _f, _f, _f,
                                ctypes.POINTER(_f)]),
     "pm_setup_proposal": (_i, [_p, _p]),

@@ -1,8 +1,8 @@
 // pm_net.hip -- gfx950 kernels of the plane-proposal network: a 3x3
 // convolution on bf16 NHWC activations as an implicit GEMM on the matrix
-// cores (v_mfma_f32_16x16x32_bf16, fp32 accumulation), its weight gradient (the
-// same instruction), and the pooling, gradient routing, loss, Adam and input
-// packing kernels of a U-Net training step.
+// cores (v_mfma_f32_16x16x32_bf16, fp32 accumulation), its weight gradient
+// (v_mfma_f32_16x16x4_f32), and the pooling, gradient routing, loss, Adam and
+// input packing kernels of a U-Net training step.
 #include <algorithm>
 #include <cstdint>
 
@@ -544,233 +544,387 @@ hipError_t launch_conv(hipStream_t st, const ConvArgs& a) {
 // ---------------------------------------------------------------------
 // weight gradient on the matrix cores: dw[co][tap, ci] = sum over pixels p
 // of g[p][co] x[p + tap][ci], a GEMM whose contraction runs over the
-// pixels.  A work-group owns 16 kM output channels x 32 input channels x
-// the 9 taps and walks 64 x 4 pixel tiles (tile t, t + splits, ...),
-// keeping the sums in accumulators; one atomic add per sum at the end.
+// pixels.
 //
-// Layout.  A matrix-core operand wants 8 contraction indices (pixels) of
-// one channel in a lane, the activations are NHWC.  A thread therefore
-// reads 8 pixels x 8 channels (8 loads of 16 bytes), transposes them in
-// registers (one v_perm_b32 per output dword) and writes 8 x 16 bytes to
-// LDS, one per channel.  The order of the contraction is free as long as
-// both operands share it, so the 8 pixels of such a unit are chosen for
-// the taps' sake: unit u of a row holds pixels u + 8 j (dilation 8: 8 u +
-// j), so a horizontal tap is another unit, never a shift inside one, and
-// the four lane groups of an operand are the tile's four rows, so a
-// vertical tap is another LDS row.  Unit u of the gradient meets units u -
-// d, u, u + d of the input: walking u, every input operand read from LDS
-// serves three taps.  The 16-byte slot of channel c of group cg in unit u
-// is c ^ ((u + 2 cg) & 7): the 8 threads that write together hit distinct
-// banks, and so do the 16 lanes that read together.
+// The order of the sum is part of the kernel.  Adam's first steps take the
+// sign of a gradient, so where one is about zero another rounding of it
+// moves the weight the other way and the next step sees another network:
+// with the bf16 instruction, which adds up 32 products at a time, and
+// gradients as near to 64-bit sums as before (3.4e-7 to 6.1e-7), the second
+// step's were 2e-4 away from those of the kernel before it.  So a sum is
+// what it was with one fmaf per pixel: kWgChunk pixels in order, in fp32.
+// v_mfma_f32_16x16x4_f32 gives exactly that chain (checked on the card:
+// no element of 64 products differs, denormals included), a product of two
+// bf16 is exact, and a pixel beyond the image or the chunk adds a zero.
+// The chunks' sums are added up in their order, in fp32, which also makes a
+// step repeatable bit for bit.  That kernel added them up with atomics as
+// they came, nearly in order: over 40 seeds its second and third step's
+// gradients differ from themselves by a median of 2.0e-7 and by more than
+// 2e-5 for 2 and 5 seeds (a weight went the other way), and from these by
+// 2.0e-7 and for 2 and 5.  Added up in 64 bits they differ by 7.1e-7, and for
+// 3 and 10 seeds.
 //
-// Bound: matrix-core issue and the LDS reads beside it (per unit and
-// wavefront 9 kM / 2 MFMAs of 16 cycles for 3 + kM / 2 reads of 1 KiB).
-// Measured against an fp32 VALU kernel that multiplied and accumulated the
-// same bf16 operands a pixel at a time: a training step on 8 pairs of 512 x
-// 384 (449 GFLOP of weight gradients) 29.0 -> 7.1 ms, its gradient as far
-// from 64-bit sums as before.
+// Layout.  A wavefront owns one chunk, 32 output channels (16 for the
+// head) and kTiles tiles of 32 k = (tap, ci).  The activations are NHWC:
+// lane 16 kk + i reads the bf16 pair of channels 2 i, 2 i + 1 of the step's
+// pixel kk, which as two fp32 are its operands of two matrix tiles, the
+// even and the odd channels.  So a step of 4 pixels is kTiles + 1 loads of
+// 4 bytes a lane, kWgAhead steps in flight, for 4 kTiles instructions of
+// 32 cycles: no LDS, no barrier.  Where the inputs' channels are multiples
+// of 32, a tile is one tap of one input and its address is scalar work; a
+// step with a tap outside the image selects each lane's address.
+// Bound: the SIMDs' fp32 units, which this instruction shares with vector
+// instructions (matrix pipe 67 % busy, vector issue 24 %; 157 TFLOP/s
+// nominal, 76-97 reached from 96 channels on).  A training step on 8 pairs of
+// 512 x 384 (449 GFLOP here): 29.0 ms with one fmaf at a time, 8.6 with this;
+// 3.9 with the bf16 instruction.
 // ---------------------------------------------------------------------
-constexpr int kWgRows = 4, kWgCols = 64;
-constexpr int kWgCi = 32;
+constexpr int kWgChunk = 1024;
+constexpr int kWgAhead = 4;
 
-// input rows and units a tile stages at dilation d: row r + dy d, unit u +
-// dx d of a 64-pixel row (dilation 8: the unit is 8 adjacent pixels)
-constexpr int wg_rows(int d) { return kWgRows + 2 * (d < 4 ? d : 4); }
-constexpr int wg_row_step(int d) { return d < 4 ? d : 4; }
-constexpr int wg_unit_step(int d) { return d == 8 ? 1 : d; }
-constexpr int wg_units(int d) { return 8 + 2 * wg_unit_step(d); }
+// what a lane reads for a pixel outside the image
+__device__ const uint32_t g_zero_pair = 0u;
 
-__device__ __forceinline__ int wg_slot(int c, int unit) {
-  const int cg = c >> 3;
-  return cg * 8 + ((c & 7) ^ ((unit + 2 * cg) & 7));
+// a pair of channels, the memory's address space in the type: a read from
+// one of two pointers stays a global one
+typedef const __attribute__((address_space(1))) uint32_t* PairPtr;
+__device__ __forceinline__ PairPtr pair_at(const void* p) {
+  return (PairPtr)(p);
 }
 
-// transposes v[pixel] (8 channels each) into 8 channels' 8 pixels and
-// stores channel c of group cg at its slot of `dst` (the unit's channels)
-__device__ __forceinline__ void wg_store(uint4* dst, int cg, int unit,
-                                         const uint4 (&v)[8]) {
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;
-    uint32_t o[4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const uint4 lo = v[2 * m], hi = v[2 * m + 1];
-      const uint32_t l = c < 2 ? lo.x : c < 4 ? lo.y : c < 6 ? lo.z : lo.w;
-      const uint32_t h = c < 2 ? hi.x : c < 4 ? hi.y : c < 6 ? hi.z : hi.w;
-      o[m] = __builtin_amdgcn_perm(h, l, sel);
-    }
-    dst[wg_slot(cg * 8 + c, unit)] = make_uint4(o[0], o[1], o[2], o[3]);
-  }
+__device__ __forceinline__ float bf16_lo(uint32_t v) {
+  return __uint_as_float(v << 16);
+}
+__device__ __forceinline__ float bf16_hi(uint32_t v) {
+  return __uint_as_float(v & 0xffff0000u);
 }
 
-template <int kM, int kDil>
-__global__ void __launch_bounds__(256, kDil <= 2 ? 2 : 1)
-k_conv_wgrad(ConvArgs a, const bf16* __restrict__ g, float* __restrict__ dw,
-             float* __restrict__ db, int tiles_x, int tiles_y, int tiles) {
-  constexpr int kCo = 16 * kM;
-  constexpr int kMW = kM / 2;             // co tiles of a wavefront
-  constexpr int kXR = wg_rows(kDil), kXU = wg_units(kDil);
-  constexpr int kUS = kDil == 8 ? 8 : 1;  // pixels between units
-  constexpr int kES = kDil == 8 ? 1 : 8;  // pixels between a unit's elements
-  constexpr int kXTasks = kXR * kXU * (kWgCi / 8);
-  constexpr int kGTasks = kWgRows * 8 * (kCo / 8);
-  __shared__ uint4 sx[kXR * kXU * kWgCi];
-  __shared__ uint4 sg[kWgRows * 8 * kCo];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int row = lane & 15, grp = lane >> 4;
-  const int wm = wave & 1, wn = wave >> 1;  // this wavefront's co, ci half
-  const int cin = a.c1 + a.c2, kpad = conv_kpad(cin);
-  const int ci0 = blockIdx.x * kWgCi, co0 = blockIdx.y * kCo;
-  const int H2 = a.up2 ? (a.H + 1) >> 1 : a.H;
-  const int W2 = a.up2 ? (a.W + 1) >> 1 : a.W;
-  const bool bias = db != nullptr && blockIdx.x == 0 && wn == 0;
-
-  f32x4 acc[kMW][9], accb[kMW];
-#pragma unroll
-  for (int m = 0; m < kMW; ++m) {
-    accb[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < 9; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  bf16x8 ones;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) ones[i] = (bf16)1.0f;
-
-  for (int t = blockIdx.z; t < tiles; t += gridDim.z) {
-    const int tx = t % tiles_x, t2 = t / tiles_x;
-    const int ty = t2 % tiles_y, n = t2 / tiles_y;
-    const int x0 = tx * kWgCols, y0 = ty * kWgRows;
-    __syncthreads();  // the previous tile's operands are read
-    for (int q = tid; q < kXTasks; q += 256) {
-      const int cg = q & 3, u = (q >> 2) % kXU, r = (q >> 2) / kXU;
-      // rows come in the three groups of the taps when they do not overlap
-      const int yy = kDil <= 4 ? y0 + r - kDil
-                               : y0 + (r & 3) + ((r >> 2) - 1) * kDil;
-      const int xb = x0 + (u - wg_unit_step(kDil)) * kUS;
-      const int c = ci0 + 8 * cg;
-      const bool rok = yy >= 0 && yy < a.H && c < cin;
-      uint4 v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int xx = xb + j * kES;
-        v[j] = make_uint4(0u, 0u, 0u, 0u);
-        if (rok && xx >= 0 && xx < a.W) {
-          if (c < a.c1) {
-            v[j] = *reinterpret_cast<const uint4*>(
-                a.x1 + (((size_t)n * a.H + yy) * a.W + xx) * a.c1 + c);
-          } else {
-            const int y2 = a.up2 ? yy >> 1 : yy, x2 = a.up2 ? xx >> 1 : xx;
-            v[j] = *reinterpret_cast<const uint4*>(
-                a.x2 + (((size_t)n * H2 + y2) * W2 + x2) * a.c2 +
-                (c - a.c1));
-          }
-        }
-      }
-      wg_store(sx + (r * kXU + u) * kWgCi, cg, u, v);
-    }
-    for (int q = tid; q < kGTasks; q += 256) {
-      const int cg = q % (kCo / 8), u = (q / (kCo / 8)) & 7;
-      const int r = q / (kCo / 8) / 8;
-      const int yy = y0 + r, xb = x0 + u * kUS, c = co0 + 8 * cg;
-      const bool rok = yy < a.H && c < a.cout;
-      uint4 v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int xx = xb + j * kES;
-        v[j] = make_uint4(0u, 0u, 0u, 0u);
-        if (rok && xx < a.W)
-          v[j] = *reinterpret_cast<const uint4*>(
-              g + (((size_t)n * a.H + yy) * a.W + xx) * a.cout + c);
-      }
-      wg_store(sg + (r * 8 + u) * kCo, cg, u, v);
-    }
-    __syncthreads();
-    // input operand of vertical tap dy at unit v (0 .. kXU - 1)
-    auto load_x = [&](int dy, int v) {
-      const int r = grp + dy * wg_row_step(kDil);
-      return __builtin_bit_cast(
-          bf16x8, sx[(r * kXU + v) * kWgCi + wg_slot(wn * 16 + row, v)]);
-    };
-    constexpr int kS = wg_unit_step(kDil);
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      bf16x8 A[kMW];
-#pragma unroll
-      for (int m = 0; m < kMW; ++m)
-        A[m] = __builtin_bit_cast(
-            bf16x8, sg[(grp * 8 + u) * kCo +
-                       wg_slot((wm * kMW + m) * 16 + row, u)]);
-#pragma unroll
-      for (int dy = 0; dy < 3; ++dy)
-#pragma unroll
-        for (int dx = 0; dx < 3; ++dx) {
-          const bf16x8 B = load_x(dy, u + dx * kS);
-#pragma unroll
-          for (int m = 0; m < kMW; ++m)
-            acc[m][3 * dy + dx] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                A[m], B, acc[m][3 * dy + dx], 0, 0, 0);
-        }
-      if (bias) {
-#pragma unroll
-        for (int m = 0; m < kMW; ++m)
-          accb[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], ones,
-                                                            accb[m], 0, 0, 0);
-      }
+// The 4 pixels of a step: the first one's index, column, row in the batch
+// and row in the image (uniform).
+struct WgStep {
+  int p, x, yrow, y;
+  __device__ __forceinline__ void next(const ConvArgs& a) {
+    p += 4;
+    x += 4;
+    while (x >= a.W) {
+      x -= a.W;
+      ++yrow;
+      if (++y == a.H) y = 0;
     }
   }
-  // a lane holds output channels 4 grp .. 4 grp + 3, input channel `row`
-  const int ci = ci0 + wn * 16 + row;
+  // pixel kk's column, row in the batch and in the image
+  __device__ __forceinline__ void lane(const ConvArgs& a, int kk, int* xl,
+                                       int* rl, int* yl) const {
+    *xl = x + kk;
+    *rl = yrow;
+    *yl = y;
+    while (*xl >= a.W) {
+      *xl -= a.W;
+      ++*rl;
+      if (++*yl == a.H) *yl = 0;
+    }
+  }
+};
+
+// the loads of a tile's steps; k0: the tile's first k
+// any channels (even), neither input upsampled
+struct WgTileAny {
+  const bf16* xp;
+  int dy, dx, c;
+  bool real;
+  __device__ __forceinline__ void init(const ConvArgs& a, int k0, int kk,
+                                       int i, int pb) {
+    const int cin = a.c1 + a.c2, k = k0 + 2 * i;
+    const int tap = k / cin, ci = k - tap * cin;
+    const bool second = ci >= a.c1;
+    c = second ? a.c2 : a.c1;
+    // k beyond the real ones: sums that nothing reads, of the pixel itself
+    real = tap < 9;
+    dy = real ? (tap / 3 - 1) * a.dil : 0;
+    dx = real ? (tap % 3 - 1) * a.dil : 0;
+    xp = second ? a.x2 + (ci - a.c1) : a.x1 + ci;
+    xp += ((ptrdiff_t)(pb + kk) + (ptrdiff_t)dy * a.W + dx) * c;
+  }
+  __device__ __forceinline__ PairPtr inner(const ConvArgs&, const WgStep&, int,
+                                           int) const {
+    return pair_at(xp);
+  }
+  __device__ __forceinline__ PairPtr outer(const ConvArgs&, int, int, int,
+                                           int) const {
+    return pair_at(xp);
+  }
+  __device__ __forceinline__ void next() { xp += 4 * c; }
+};
+
+// c1 and c2 multiples of 32: all but the lane's channel pair is uniform
+struct WgTile32 {
+  const bf16* xp;  // channel 0 of the tile at the step's first pixel's tap,
+                   // or, upsampled, at the input's first pixel
+  int dy, dx, c;
+  bool up;
+  static constexpr bool real = true;
+  __device__ __forceinline__ void init(const ConvArgs& a, int k0, int, int,
+                                       int pb) {
+    const int cin = a.c1 + a.c2;
+    const int tap = k0 / cin, ci = k0 - tap * cin;
+    const bool second = ci >= a.c1;
+    c = second ? a.c2 : a.c1;
+    dy = (tap / 3 - 1) * a.dil;
+    dx = (tap % 3 - 1) * a.dil;
+    up = second && a.up2;
+    xp = second ? a.x2 + (ci - a.c1) : a.x1 + ci;
+    if (!up) xp += ((ptrdiff_t)pb + (ptrdiff_t)dy * a.W + dx) * c;
+  }
+  // H and W are even where x2 is upsampled, so the batch's rows halve as
+  // the image's do
+  __device__ __forceinline__ PairPtr inner(const ConvArgs& a, const WgStep& s,
+                                           int kk, int i) const {
+    if (!up) return pair_at(xp + (unsigned)(kk * c + 2 * i));
+    const int col = s.x + dx;
+    const bf16* q =
+        xp + ((size_t)((s.yrow + dy) >> 1) * (a.W >> 1) + (col >> 1)) * c;
+    return pair_at(q + (unsigned)(((kk + (col & 1)) >> 1) * c + 2 * i));
+  }
+  __device__ __forceinline__ PairPtr outer(const ConvArgs& a, int xl, int rl,
+                                           int kk, int i) const {
+    if (!up) return pair_at(xp + (unsigned)(kk * c + 2 * i));
+    return pair_at(xp +
+                   ((ptrdiff_t)((rl + dy) >> 1) * (a.W >> 1) +
+                    ((xl + dx) >> 1)) * c + 2 * i);
+  }
+  __device__ __forceinline__ void next() { xp += up ? 0 : 4 * c; }
+};
+
+// part: per chunk its sums, [cpad][kpad], and after those of all chunks
+// their bias sums, [cpad] per chunk.  kCT: matrix tiles of output channels.
+template <int kCT, int kTiles, typename Tile>
+__global__ void __launch_bounds__(256)
+k_conv_wgrad(ConvArgs a, const bf16* __restrict__ g, float* __restrict__ part,
+             bool with_bias, int groups, int cts, int chunks) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int i = lane & 15, kk = lane >> 4;
+  // each XCD takes a run of units, which share their pixels in its L2
+  const unsigned per = gridDim.x / 8;
+  const unsigned unit =
+      (blockIdx.x % 8 * per + blockIdx.x / 8) * 4 + (unsigned)wave;
+  if (unit >= (unsigned)groups * cts * chunks) return;
+  const int kg = (int)(unit % groups), ct = (int)(unit / groups % cts);
+  const int chunk = (int)(unit / groups / cts);
+  const int cin = a.c1 + a.c2, kpad = conv_kpad(cin), cpad = conv_cpad(a.cout);
+  const int npix = a.N * a.H * a.W;
+  const int pb = chunk * kWgChunk;
+  const int pe = std::min(npix - pb, kWgChunk) + pb;
+  const PairPtr zero = pair_at(&g_zero_pair);
+
+  WgStep s;
+  s.p = pb;
+  s.yrow = pb / a.W;
+  s.x = pb - s.yrow * a.W;
+  s.y = s.yrow % a.H;
+  // this lane's channels of g; rows beyond cout are sums that nothing reads
+  const int co = 32 * ct + (kCT == 2 ? 2 * i : i & ~1);
+  const unsigned gl = (unsigned)(kk * a.cout + std::min(co, a.cout - 2));
+  const bf16* gp = g + (size_t)pb * a.cout;
+  Tile tile[kTiles];
 #pragma unroll
-  for (int m = 0; m < kMW; ++m)
+  for (int t = 0; t < kTiles; ++t)
+    tile[t].init(a, 32 * (kTiles * kg + t), kk, i, pb);
+
+  typedef uint32_t Pairs[kTiles + 1];
+  auto issue = [&](Pairs& r) {
+    // addresses on both sides of the branch, the loads after it: so each
+    // wait counts the loads issued since
+    PairPtr q[kTiles + 1];
+    if (s.p + 4 <= pe && s.x >= a.dil && s.x + 4 + a.dil <= a.W &&
+        s.y >= a.dil && s.y + a.dil < a.H) {
+      q[0] = pair_at(gp + gl);
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) q[t + 1] = tile[t].inner(a, s, kk, i);
+    } else {
+      int xl, rl, yl;
+      s.lane(a, kk, &xl, &rl, &yl);
+      const bool there = s.p + kk < pe;
+      q[0] = there ? pair_at(gp + gl) : zero;
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) {
+        const bool ok = there && tile[t].real &&
+                        (unsigned)(yl + tile[t].dy) < (unsigned)a.H &&
+                        (unsigned)(xl + tile[t].dx) < (unsigned)a.W;
+        q[t + 1] = tile[t].outer(a, xl, rl, kk, i);
+        q[t + 1] = ok ? q[t + 1] : zero;
+      }
+    }
+#pragma unroll
+    for (int t = 0; t <= kTiles; ++t) r[t] = *q[t];
+    gp += 4 * a.cout;
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) tile[t].next();
+    s.next(a);
+  };
+
+  f32x4 acc[kTiles][kCT][2], accb[kCT];
+#pragma unroll
+  for (int c = 0; c < kCT; ++c) {
+    accb[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+      acc[t][c][0] = acc[t][c][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const bool bias = with_bias && kg == 0;
+  auto consume = [&](const Pairs& r) {
+    float A[kCT];
+    if (kCT == 2) {
+      A[0] = bf16_lo(r[0]);
+      A[kCT - 1] = bf16_hi(r[0]);
+    } else {
+      A[0] = i & 1 ? bf16_hi(r[0]) : bf16_lo(r[0]);
+    }
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      const float B[2] = {bf16_lo(r[t + 1]), bf16_hi(r[t + 1])};
+#pragma unroll
+      for (int c = 0; c < kCT; ++c)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          acc[t][c][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              A[c], B[e], acc[t][c][e], 0, 0, 0);
+    }
+    if (bias) {
+#pragma unroll
+      for (int c = 0; c < kCT; ++c)
+        accb[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[c], 1.0f, accb[c], 0,
+                                                       0, 0);
+    }
+  };
+
+  Pairs raw[kWgAhead];
+#pragma unroll
+  for (int d = 0; d < kWgAhead; ++d) issue(raw[d]);
+  for (int q = pb; q < pe; q += 4 * kWgAhead) {
+#pragma unroll
+    for (int d = 0; d < kWgAhead; ++d) {
+      consume(raw[d]);
+      issue(raw[d]);  // of pixels beyond the chunk: zeros
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  // a lane holds rows 4 kk .. 4 kk + 3 of column i of every tile
+  float* const out = part + (size_t)chunk * cpad * kpad;
+  float* const outb =
+      part + (size_t)chunks * cpad * kpad + (size_t)chunk * cpad;
+#pragma unroll
+  for (int c = 0; c < kCT; ++c)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int co = co0 + (wm * kMW + m) * 16 + 4 * grp + j;
-      if (co >= a.cout) continue;
-      if (ci < cin)
+      const int row = 32 * ct + (kCT == 2 ? 2 * (4 * kk + j) + c : 4 * kk + j);
 #pragma unroll
-        for (int t = 0; t < 9; ++t)
-          atomicAdd(&dw[(size_t)co * kpad + t * cin + ci], acc[m][t][j]);
-      if (bias && row == 0) atomicAdd(&db[co], accb[m][j]);
+      for (int t = 0; t < kTiles; ++t) {
+        const int k = 32 * (kTiles * kg + t) + 2 * i;
+        if (k < kpad)
+          *reinterpret_cast<float2*>(out + (size_t)row * kpad + k) =
+              make_float2(acc[t][c][0][j], acc[t][c][1][j]);
+      }
+      if (bias && i == 0) outb[row] = accb[c][j];
     }
 }
 
-constexpr unsigned kWgGroups = 512;
+// The chunks' sums added up in order, 64 elements per work-group: 16
+// wavefronts fetch kWgFetch chunks each ahead, the first adds.
+constexpr int kWgSums = 16, kWgFetch = 8;
 
-template <int kM, int kDil>
-static hipError_t launch_wgrad_tile(hipStream_t st, const ConvArgs& a,
-                                    const bf16* g, float* dw, float* db) {
-  const int tiles_x = (a.W + kWgCols - 1) / kWgCols;
-  const int tiles_y = (a.H + kWgRows - 1) / kWgRows;
-  const long tiles = (long)tiles_x * tiles_y * a.N;
-  const unsigned nci = (unsigned)((a.c1 + a.c2 + kWgCi - 1) / kWgCi);
-  const unsigned nco = (unsigned)((a.cout + 16 * kM - 1) / (16 * kM));
-  // two work-groups per CU in all: each ends with one atomic add per sum,
-  // so no more splits of the pixels than fill the GPU
-  const long splits =
-      std::min<long>(tiles, std::max<long>(1, kWgGroups / (nci * nco)));
-  NET_LAUNCH((k_conv_wgrad<kM, kDil>), dim3(nci, nco, (unsigned)splits),
-             dim3(256), 0, st, a, g, dw, db, tiles_x, tiles_y, (int)tiles);
+__global__ void __launch_bounds__(64 * kWgSums)
+k_wgrad_sum(const float* __restrict__ part, int chunks, int cout, int cpad,
+            int kpad, int kreal, int wblocks, float* __restrict__ dw,
+            float* __restrict__ db) {
+  constexpr int kBatch = kWgSums * kWgFetch;
+  __shared__ float sums[kBatch][64];
+  const int tx = threadIdx.x, ty = threadIdx.y;
+  const bool bias = (int)blockIdx.x >= wblocks;
+  const int e = ((int)blockIdx.x - (bias ? wblocks : 0)) * 64 + tx;
+  const size_t stride = bias ? (size_t)cpad : (size_t)cpad * kpad;
+  const float* src =
+      part + (bias ? (size_t)chunks * cpad * kpad : (size_t)0) + e;
+  const bool real = bias ? e < cout : e < cout * kpad && e % kpad < kreal;
+  float s = 0.0f;
+  for (int c0 = 0; c0 < chunks; c0 += kBatch) {
+    float v[kWgFetch];
+#pragma unroll
+    for (int u = 0; u < kWgFetch; ++u) {
+      const int c = c0 + ty + kWgSums * u;
+      v[u] = real && c < chunks ? src[c * stride] : 0.0f;
+    }
+    __syncthreads();  // the batch before is added up
+#pragma unroll
+    for (int u = 0; u < kWgFetch; ++u) sums[ty + kWgSums * u][tx] = v[u];
+    __syncthreads();
+    if (ty == 0) {
+      const int n = std::min(chunks - c0, kBatch);
+#pragma unroll 8
+      for (int c = 0; c < n; ++c) s += sums[c][tx];
+    }
+  }
+  if (ty == 0 && real) (bias ? db : dw)[e] = s;
 }
 
-template <int kDil>
-static hipError_t launch_wgrad_dil(hipStream_t st, const ConvArgs& a,
-                                   const bf16* g, float* dw, float* db) {
-  // 64 output channels per work-group halve the input reads per product
-  if (a.cout % 64 == 0) return launch_wgrad_tile<4, kDil>(st, a, g, dw, db);
-  return launch_wgrad_tile<2, kDil>(st, a, g, dw, db);
+static int wgrad_chunks(int N, int H, int W) {
+  return (int)(((long)N * H * W + kWgChunk - 1) / kWgChunk);
+}
+
+size_t wgrad_part_floats(int N, int H, int W, int cin, int cout) {
+  return (size_t)wgrad_chunks(N, H, W) * conv_cpad(cout) *
+         (conv_kpad(cin) + 1);
+}
+
+template <int kCT, int kTiles, typename Tile>
+static hipError_t launch_wgrad_chains(hipStream_t st, const ConvArgs& a,
+                                      const bf16* g, float* part,
+                                      bool with_bias) {
+  const int chunks = wgrad_chunks(a.N, a.H, a.W);
+  const int tiles = conv_kpad(a.c1 + a.c2) / 32;
+  const int groups = (tiles + kTiles - 1) / kTiles;
+  const int cts = conv_cpad(a.cout) / 32;
+  const long units = (long)groups * cts * chunks;
+  NET_LAUNCH((k_conv_wgrad<kCT, kTiles, Tile>),
+             dim3((unsigned)((units + 31) / 32 * 8)), dim3(256), 0, st, a, g,
+             part, with_bias, groups, cts, chunks);
+}
+
+template <int kCT>
+static hipError_t launch_wgrad_tiles(hipStream_t st, const ConvArgs& a,
+                                     const bf16* g, float* part,
+                                     bool with_bias) {
+  if (a.c1 % 32 || a.c2 % 32)
+    return launch_wgrad_chains<kCT, 3, WgTileAny>(st, a, g, part, with_bias);
+  // Three tiles share a step's gradients.  Below 1.5 wavefronts per SIMD that
+  // way (the 8 x 48 x 64 layers of a training batch: 864 and 1152), one tile
+  // each leaves fewer of them with a second round: dilation 2, 4, 8 161 / 166
+  // / 178 -> 120 / 122 / 129 us.  At 2592 it is even (214), at 4608 slower
+  // (341 -> 373).
+  const long units = (long)wgrad_chunks(a.N, a.H, a.W) *
+                     (conv_cpad(a.cout) / 32) *
+                     (conv_kpad(a.c1 + a.c2) / 96);
+  if (units < 1536)
+    return launch_wgrad_chains<kCT, 1, WgTile32>(st, a, g, part, with_bias);
+  return launch_wgrad_chains<kCT, 3, WgTile32>(st, a, g, part, with_bias);
 }
 
 hipError_t launch_conv_wgrad(hipStream_t st, const ConvArgs& a, const bf16* g,
-                             float* dw, float* db) {
-  switch (a.dil) {
-    case 1: return launch_wgrad_dil<1>(st, a, g, dw, db);
-    case 2: return launch_wgrad_dil<2>(st, a, g, dw, db);
-    case 4: return launch_wgrad_dil<4>(st, a, g, dw, db);
-    case 8: return launch_wgrad_dil<8>(st, a, g, dw, db);
-  }
-  return hipErrorInvalidValue;
+                             float* part, float* dw, float* db) {
+  if (a.c1 % 2 || a.c2 % 2 || a.cout % 2 ||
+      (a.up2 && (a.H % 2 || a.W % 2 || a.c1 % 32 || a.c2 % 32)))
+    return hipErrorInvalidValue;
+  const hipError_t e =
+      a.cout <= 16 ? launch_wgrad_tiles<1>(st, a, g, part, db != nullptr)
+                   : launch_wgrad_tiles<2>(st, a, g, part, db != nullptr);
+  if (e != hipSuccess) return e;
+  const int cpad = conv_cpad(a.cout), kpad = conv_kpad(a.c1 + a.c2);
+  const int wblocks = (a.cout * kpad + 63) / 64;
+  const int bblocks = db ? (a.cout + 63) / 64 : 0;
+  NET_LAUNCH(k_wgrad_sum, dim3((unsigned)(wblocks + bblocks)),
+             dim3(64, kWgSums), 0, st, part, wgrad_chunks(a.N, a.H, a.W),
+             a.cout, cpad, kpad, 9 * (a.c1 + a.c2), wblocks, dw, db);
 }
 
 // ---------------------------------------------------------------------

@@ -103,6 +103,7 @@ struct pm_net {
   DevBuf gact[kTensors];  // of the pooled tensors and their pools only
   DevBuf tmp;        // gradient of an upsampled input before its sum (fp32)
   DevBuf gz[2];      // masked output gradients (bf16): a layer's, the next's
+  DevBuf wpart;      // a weight gradient's sums before the last addition
   DevBuf loss;       // one float
   int N = 0, H = 0, W = 0;
 };
@@ -182,6 +183,18 @@ int alloc_batch(pm_net* n, int N, int H, int W) {
   n->H = H;
   n->W = W;
   return PM_OK;
+}
+
+// the training step's own: a forward pass does without
+int alloc_wpart(pm_net* n) {
+  size_t floats = 0;
+  for (int l = 0; l < kConvs; ++l) {
+    const int lev = kT[kC[l].out].level;
+    floats = std::max(floats, pm::net::wgrad_part_floats(
+                                  n->N, n->H >> lev, n->W >> lev, conv_cin(l),
+                                  conv_cout(l)));
+  }
+  return ensure(n, n->wpart, floats * sizeof(float));
 }
 
 pm::net::ConvArgs conv_args(pm_net* n, int l) {
@@ -282,7 +295,7 @@ int backward(pm_net* n, hipStream_t st) {
     const int l = op;
     const ConvDesc& d = kC[l];
     pm::net::ConvArgs a = conv_args(n, l);
-    NET_HIP(n, pm::net::launch_conv_wgrad(st, a, gz,
+    NET_HIP(n, pm::net::launch_conv_wgrad(st, a, gz, as<float>(n->wpart),
                                           as<float>(n->grad) + n->woff[l],
                                           as<float>(n->grad) + n->boff[l]));
     if (d.in1 == X0) continue;  // the input needs no gradient
@@ -445,7 +458,7 @@ void pm_net_destroy(pm_net* n) {
   (void)hipSetDevice(n->device);
   if (n->stream) (void)hipStreamSynchronize(n->stream);
   DevBuf* bufs[] = {&n->w32, &n->w16, &n->grad, &n->m, &n->v, &n->tmp,
-                    &n->gz[0], &n->gz[1], &n->loss};
+                    &n->gz[0], &n->gz[1], &n->wpart, &n->loss};
   for (DevBuf* b : bufs)
     if (b->ptr) (void)hipFree(b->ptr);
   for (int t = 0; t < kTensors; ++t) {
@@ -525,13 +538,13 @@ int pm_net_train_step(pm_net* n, const float* d_x, const float* d_target,
   int rc;
   if ((rc = check_dims(n, N, H, W))) return rc;
   NET_HIP(n, hipSetDevice(n->device));
-  if ((rc = alloc_batch(n, N, H, W))) return rc;
+  if ((rc = alloc_batch(n, N, H, W)) || (rc = alloc_wpart(n))) return rc;
   hipStream_t st = n->stream;
   const size_t npix = (size_t)N * H * W;
   NET_HIP(n, pm::net::launch_to_bf16(st, npix * PM_NET_IN_CHANNELS, d_x,
                                      as<bf16>(n->act[X0])));
   if ((rc = forward(n, st))) return rc;
-  // parameter gradients are accumulated over the pixels
+  // the padding of the parameter gradients stays zero
   NET_HIP(n, hipMemsetAsync(n->grad.ptr, 0, n->nparams * 4, st));
   NET_HIP(n, hipMemsetAsync(n->loss.ptr, 0, 4, st));
   NET_HIP(n, pm::net::launch_l1_loss(st, npix, as<float>(n->act[OUT]),
@@ -552,6 +565,56 @@ int pm_net_train_step(pm_net* n, const float* d_x, const float* d_target,
   if (loss) {
     NET_HIP(n, hipMemcpyAsync(loss, n->loss.ptr, 4, hipMemcpyDeviceToHost, st));
     NET_HIP(n, hipStreamSynchronize(st));
+  }
+  return PM_OK;
+}
+
+int pm_net_conv_selftest(pm_net* n, const void* d_x1, int c1,
+                         const void* d_x2, int c2, int up2, int N, int H,
+                         int W, int cout, int dil, const void* d_w,
+                         float* d_y, const void* d_g, float* d_dw,
+                         float* d_db) {
+  if (!n) return PM_ERR_ARG;
+  if (!d_x1 || (c2 > 0 && !d_x2) || (d_y && !d_w) || (d_dw && !d_g) ||
+      (d_db && !d_dw))
+    return fail(n, PM_ERR_ARG, "NULL buffer");
+  if (c1 < 8 || c1 % 8 || c2 < 0 || c2 % 8 || cout < 8 || cout % 8)
+    return fail(n, PM_ERR_ARG, "channels must be multiples of 8");
+  if (N < 1 || H < 1 || W < 1 || (long)N * H * W > (1L << 27))
+    return fail(n, PM_ERR_ARG, "size %d x %d x %d", N, H, W);
+  if (up2 && (H % 2 || W % 2 || c1 % 32 || c2 % 32))
+    return fail(n, PM_ERR_ARG, "an upsampled input needs an even size and "
+                "channels in multiples of 32");
+  if (dil != 1 && dil != 2 && dil != 4 && dil != 8)
+    return fail(n, PM_ERR_ARG, "dilation %d", dil);
+  for (const void* p : {d_x1, d_x2, d_w, d_g, (const void*)d_y,
+                        (const void*)d_dw, (const void*)d_db})
+    if (reinterpret_cast<uintptr_t>(p) % 16)
+      return fail(n, PM_ERR_ARG, "buffers must be aligned to 16 bytes");
+  NET_HIP(n, hipSetDevice(n->device));
+  pm::net::ConvArgs a;
+  a.x1 = static_cast<const bf16*>(d_x1);
+  a.x2 = static_cast<const bf16*>(d_x2);
+  a.c1 = c1;
+  a.c2 = c2;
+  a.up2 = up2;
+  a.w = static_cast<const bf16*>(d_w);
+  a.N = N;
+  a.H = H;
+  a.W = W;
+  a.cout = a.ys = cout;
+  a.dil = dil;
+  a.yf = d_y;
+  if (d_y) NET_HIP(n, pm::net::launch_conv(n->stream, a));
+  if (d_dw) {
+    int rc;
+    if ((rc = ensure(n, n->wpart,
+                     pm::net::wgrad_part_floats(N, H, W, c1 + c2, cout) *
+                         sizeof(float))))
+      return rc;
+    NET_HIP(n, pm::net::launch_conv_wgrad(n->stream, a,
+                                          static_cast<const bf16*>(d_g),
+                                          as<float>(n->wpart), d_dw, d_db));
   }
   return PM_OK;
 }

@@ -53,11 +53,17 @@ struct ConvArgs {
 };
 hipError_t launch_conv(hipStream_t st, const ConvArgs& a);
 
-// Weight gradient of the convolution above: dw[co][k] += sum over the
-// N x H x W pixels of g[p][co] * x(p, k), g bf16 with cout channels; and
-// db[co] += sum of g[p][co] when db is not null.  fp32 accumulation.
+// Weight gradient of the convolution above: dw[co][k] = sum over the
+// N x H x W pixels of g[p][co] * x(p, k), g bf16 with cout channels, for the
+// real co and k; and db[co] = sum of g[p][co] when db is not null.  The
+// pixels (image, row, column) are summed 1024 at a time, in order, with one
+// fp32 fmaf each; then those sums in order, in fp32.  c1, c2 and cout even; when up2, H
+// and W even, c1 and c2 multiples of 32.  part: wgrad_part_floats floats to
+// work in.
+size_t wgrad_part_floats(int N, int H, int W, int cin, int cout);
 hipError_t launch_conv_wgrad(hipStream_t st, const ConvArgs& a,
-                             const bf16* g, float* dw, float* db);
+                             const bf16* g, float* part, float* dw,
+                             float* db);
 
 // w'[ci][k'] for the gradient of the input: the convolution of the output
 // gradient (cout channels) with the flipped, transposed kernel, k' = (8 -

@@ -78,6 +78,23 @@ int pm_net_train_step(pm_net* net, const float* d_x, const float* d_target,
  * (n = pm_net_num_params floats, host), before its Adam update. */
 int pm_net_get_grads(pm_net* net, float* out, size_t n);
 
+/* Diagnostic: one 3x3 convolution of the network's kernels on the caller's
+ * operands, and its weight gradient.  d_x1 (N x H x W x c1 bf16) and, with
+ * c2 > 0, d_x2 (c2 channels; N x H/2 x W/2 and read nearest-upsampled with
+ * up2) are the concatenated input, zero beyond the image; channels are
+ * multiples of 8 (with up2 of 32, and H and W even), dil is 1, 2, 4 or 8,
+ * buffers are aligned to 16 bytes.  With k = (3 (dy + 1) + dx + 1) (c1 + c2) + ci, rows of
+ * kpad = 9 (c1 + c2) rounded up to 32 and cpad = cout rounded up to 32:
+ * d_y (N x H x W x cout fp32, may be NULL) = the convolution with d_w (cpad x
+ * kpad bf16, zero beyond the real ones); d_dw (cpad x kpad fp32, may be NULL;
+ * the real ones are written) and d_db (cpad fp32, may be NULL) = the sums over
+ * the pixels of g x and of g, for d_g (N x H x W x cout bf16). */
+int pm_net_conv_selftest(pm_net* net, const void* d_x1, int c1,
+                         const void* d_x2, int c2, int up2, int N, int H,
+                         int W, int cout, int dil, const void* d_w,
+                         float* d_y, const void* d_g, float* d_dw,
+                         float* d_db);
+
 /* Setup of a context seeded by the network, the counterpart of pm_setup
  * (PMHuberStereo.cpp:445-487) with init replaced by the proposal: the
  * network runs on the context's pair for the left view and on the
