@@ -54,7 +54,7 @@ struct pm_ctx {
   DevBuf state[2][2];   // [view][ping-pong]
   DevBuf vbuf[2];       // vbuf[0]: filled by the left view, vbuf[1]: right
   DevBuf flat[2];       // costs of the cleared smooth field's proposal
-  bool costs_known[2] = {};  // the plane field's cost channel can be trusted
+  DevBuf words;         // pm::CostWords of the plane fields
   DevBuf checked;       // LR-checked left field
   DevBuf scratch4;      // W*H float4 (host transfers, normals)
   DevBuf scratch4b;     // W*H float4
@@ -204,6 +204,7 @@ int alloc_pair(pm_ctx* c, int W, int H, int channels) {
         (rc = ensure(c, c->flat[v], n * pm::kFlatCosts * sizeof(float))))
       return rc;
   }
+  if ((rc = ensure(c, c->words, sizeof(pm::CostWords)))) return rc;
   if ((rc = ensure(c, c->checked, n * sizeof(float4)))) return rc;
   if ((rc = ensure(c, c->scratch4, n * sizeof(float4)))) return rc;
   if ((rc = ensure(c, c->scratch4b, n * sizeof(float4)))) return rc;
@@ -291,6 +292,10 @@ int set_images(pm_ctx* c, const float* l, const float* r, int W, int H,
   c->ready = false;
   c->last_pp = -1;
   return PM_OK;
+}
+
+pm::CostWords* cost_words(pm_ctx* c) {
+  return static_cast<pm::CostWords*>(c->words.ptr);
 }
 
 // bilateral weights + gradients of both views (PMHuberStereo.cpp:445-450)
@@ -590,7 +595,6 @@ int one_iteration(pm_ctx* c, unsigned long long* counters, bool split,
   a.flat_known = first ? 0 : 1;
   int rc;
 
-  a.costs_known = c->costs_known[0];
   a.flat_cost = huber ? nullptr : static_cast<float*>(c->flat[0].ptr);
   a.self = view_bufs(c, 0);
   a.other = view_bufs(c, 1);
@@ -605,7 +609,6 @@ int one_iteration(pm_ctx* c, unsigned long long* counters, bool split,
   if (huber && (rc = smooth_after(c, 0, state_ptr(c, 0, nxt), theta, split)))
     return rc;
 
-  a.costs_known = c->costs_known[1];
   a.flat_cost = huber ? nullptr : static_cast<float*>(c->flat[1].ptr);
   a.self = view_bufs(c, 1);
   a.other = view_bufs(c, 0);
@@ -623,7 +626,6 @@ int one_iteration(pm_ctx* c, unsigned long long* counters, bool split,
   if (huber) {
     c->theta = theta_after(c, c->iteration, c->theta);
   }
-  c->costs_known[0] = c->costs_known[1] = true;
   c->cur = nxt;
   c->iteration += 1;
   return PM_OK;
@@ -644,6 +646,10 @@ int iterate_n(pm_ctx* c, int n, unsigned long long* counters) {
       return fail(c, PM_ERR_ARG, "pm_iterate with smoothing cannot be "
                   "recorded by stream capture");
   }
+  if (n > 0)
+    PM_HIP(c, pm::launch_forget_costs(c->stream, c->geo.npix, cost_words(c),
+                                      state_ptr(c, 0, c->cur),
+                                      state_ptr(c, 1, c->cur)));
   if (split && (rc = split_rebase(c))) return rc;
   for (int i = 0; i < n; ++i)
     if ((rc = one_iteration(c, counters, split, i == 0))) break;
@@ -826,6 +832,7 @@ void pm_destroy(pm_ctx* c) {
       release(c->rofb[v].q[k]);
     }
   }
+  release(c->words);
   release(c->checked);
   release(c->scratch4);
   release(c->scratch4b);
@@ -875,11 +882,11 @@ int pm_setup(pm_ctx* c) {
                             state_ptr(c, 1, 0)));
   PM_HIP(c, pm::launch_viewbuf_clear(
                 c->stream, c->geo,
-                static_cast<unsigned long long*>(c->vbuf[1].ptr)));
+                static_cast<unsigned long long*>(c->vbuf[1].ptr),
+                cost_words(c)));
   if ((rc = huber_setup(c))) return rc;
   c->cur = 0;
   c->iteration = 0;
-  c->costs_known[0] = c->costs_known[1] = true;
   c->ready = true;
   c->last_pp = -1;
   return PM_OK;
@@ -949,11 +956,11 @@ int pm_setup_proposal_views(pm_ctx* c, pm_net* net, int views) {
   }
   PM_HIP(c, pm::launch_viewbuf_clear(
                 c->stream, c->geo,
-                static_cast<unsigned long long*>(c->vbuf[1].ptr)));
+                static_cast<unsigned long long*>(c->vbuf[1].ptr),
+                cost_words(c)));
   if ((rc = huber_setup(c))) return rc;
   c->cur = 0;
   c->iteration = 0;
-  c->costs_known[0] = c->costs_known[1] = true;
   c->ready = true;
   c->last_pp = -1;
   return PM_OK;
@@ -983,7 +990,8 @@ int pm_setup_prior(pm_ctx* c, const float* disparity, const float* normals) {
                             state_ptr(c, 1, 0)));
   PM_HIP(c, pm::launch_viewbuf_clear(
                 c->stream, c->geo,
-                static_cast<unsigned long long*>(c->vbuf[1].ptr)));
+                static_cast<unsigned long long*>(c->vbuf[1].ptr),
+                cost_words(c)));
   if ((rc = huber_setup(c))) return rc;
   // the seeded left planes start the left smooth field
   // (PMHuberStereo.cpp:473-477)
@@ -993,7 +1001,6 @@ int pm_setup_prior(pm_ctx* c, const float* disparity, const float* normals) {
   PM_HIP(c, hipStreamSynchronize(c->stream));  // host inputs may be freed
   c->cur = 0;
   c->iteration = 0;
-  c->costs_known[0] = c->costs_known[1] = true;
   c->ready = true;
   c->last_pp = -1;
   return PM_OK;
@@ -1052,7 +1059,8 @@ int pm_set_planes(pm_ctx* c, int view, const float* in, int iteration) {
     return rc;
   if (!in) return fail(c, PM_ERR_ARG, "in is NULL");
   if (iteration < 0) return fail(c, PM_ERR_ARG, "negative iteration");
-  c->costs_known[view] = false;  // whatever the caller's cost channel holds
+  // whatever the caller's cost channel holds
+  PM_HIP(c, pm::launch_costs_unknown(c->stream, cost_words(c), view));
   if ((rc = to_device(c, state_ptr(c, view, c->cur), in,
                       c->geo.npix * sizeof(float4))))
     return rc;

@@ -90,9 +90,24 @@ struct Window {
   int left = 0, cols = 0;
 };
 
+// Whose costs the cost channels of the two plane fields hold, in device
+// memory and changed in stream order, so that a captured run sees whose
+// planes it is replayed on.
+struct CostWords {
+  uint32_t known[2];    // by view: the engine's, or NaN; 0: a caller's values
+  uint32_t tickets[2];  // launch_forget_costs's, 0 between launches
+};
+
 // before the launch_prepare of the two views
 hipError_t launch_clear_wild(hipStream_t st, const Geometry& g, ViewBufs a,
                              ViewBufs b);
+
+// view's field holds a caller's values
+hipError_t launch_costs_unknown(hipStream_t st, CostWords* cw, int view);
+
+// before a propagate: NaN, which it evaluates, for a caller's values
+hipError_t launch_forget_costs(hipStream_t st, size_t npix, CostWords* cw,
+                               float4* left, float4* right);
 
 hipError_t launch_prepare(hipStream_t st, const Geometry& g, const float* img,
                           int channels, int stride, ViewBufs v);
@@ -120,8 +135,10 @@ hipError_t launch_init_proposal(hipStream_t st, const Geometry& g,
 hipError_t launch_viewbuf_clear_rows(hipStream_t st, const Geometry& g,
                                      unsigned long long* vbuf, int row0,
                                      int rows);
+// cw (may be null): also say that the engine made both fields
 hipError_t launch_viewbuf_clear(hipStream_t st, const Geometry& g,
-                                unsigned long long* vbuf);
+                                unsigned long long* vbuf,
+                                CostWords* cw = nullptr);
 
 struct PropagateArgs {
   ViewBufs self, other;
@@ -136,10 +153,6 @@ struct PropagateArgs {
   // red-black pass 1 (Geometry::color == 1): the pass-0 pixels' new planes,
   // read instead of `old` for neighbours of colour 0 (may alias `out`)
   const float4* fresh = nullptr;
-  // the cost channel of `old` holds its planes' costs (of this cost kind,
-  // as an evaluation without an early exit gives them, or NaN, or the 1.0
-  // of the census exit)
-  int costs_known = 0;
   // without a smooth field: kFlatCosts floats per pixel for the cost of the
   // cleared field's proposal, written (flat_known = 0) or read; may be null
   float* flat_cost = nullptr;

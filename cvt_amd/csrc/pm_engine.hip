@@ -1422,6 +1422,28 @@ __global__ void k_clear_wild(uint32_t* __restrict__ a,
   if (threadIdx.x == 0) *a = *b = 0u;
 }
 
+__global__ void k_costs_unknown(CostWords* cw, int view) {
+  if (threadIdx.x == 0) cw->known[view] = 0u;
+}
+
+// The work-group that finishes last says that the field's costs are known.
+// Every work-group has read the word by then, so all find the same.
+__global__ void __launch_bounds__(256)
+k_forget_costs(size_t npix, CostWords* cw, float4* __restrict__ left,
+               float4* __restrict__ right) {
+  const int view = blockIdx.y;
+  if (cw->known[view]) return;
+  float4* s = view ? right : left;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < npix;
+       i += (size_t)gridDim.x * 256)
+    s[i].w = NAN;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  if (atomicAdd(&cw->tickets[view], 1u) != gridDim.x - 1) return;
+  cw->tickets[view] = 0u;
+  cw->known[view] = 1u;
+}
+
 __global__ void __launch_bounds__(256)
 k_prepare(const float* __restrict__ img, int W, int H, int C, int stride,
           int R, float cw, float lim, float4* __restrict__ tex,
@@ -1587,9 +1609,11 @@ k_init_from_view(int W, int H, float dmax,
 }
 
 __global__ void __launch_bounds__(256)
-k_viewbuf_clear(size_t n, unsigned long long* __restrict__ vbuf) {
+k_viewbuf_clear(size_t n, unsigned long long* __restrict__ vbuf,
+                CostWords* cw) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i < n) vbuf[i] = ~0ull;
+  if (cw && i == 0) *cw = CostWords{{1u, 1u}, {0u, 0u}};
 }
 
 // ---------------------------------------------------------------------
@@ -1696,11 +1720,12 @@ __device__ __forceinline__ void propagate_block(
     float4 cand = self;
     bool active = L.valid;
     if (k == kCandSelf) {
-      // The old plane's cost.  Where the cost channel is known to hold it
-      // (a.costs_known), only the values that do not settle it are
-      // evaluated again: NaN (no cost yet, or a colour+gradient patch
-      // without a tap) and the 1.0 of the census early exit.
-      if (!kCount && a.costs_known) {
+      // The old plane's cost.  The cost channel holds it as an evaluation
+      // without an early exit gives it, and only the values that do not
+      // settle it are evaluated again: NaN (no cost yet, or a
+      // colour+gradient patch without a tap) and the 1.0 of the census
+      // early exit.
+      if (!kCount) {
         active = active && (self.w != self.w ||
                             (kKind != kCostColorGrad && self.w == 1.0f));
         if (!__any(active)) continue;
@@ -2146,8 +2171,6 @@ __device__ __forceinline__ PropagateArgs batch_args(const BatchPair& P,
   a.theta = 0.0f;
   a.lr = view == 0 ? 1 : 0;
   a.iter = iter;
-  // every field was made by this run
-  a.costs_known = 1;
   a.flat_cost = P.flat[view];
   a.flat_known = iter > 0;
   return a;
@@ -2304,6 +2327,18 @@ hipError_t launch_clear_wild(hipStream_t st, const Geometry& g, ViewBufs a,
             wild_word(b.tex, g.TS, g.H));
 }
 
+hipError_t launch_costs_unknown(hipStream_t st, CostWords* cw, int view) {
+  PM_LAUNCH(k_costs_unknown, dim3(1), dim3(64), 0, st, cw, view);
+}
+
+hipError_t launch_forget_costs(hipStream_t st, size_t npix, CostWords* cw,
+                               float4* left, float4* right) {
+  const unsigned blocks =
+      (unsigned)std::min<size_t>((npix + 255) / 256, 256);
+  PM_LAUNCH(k_forget_costs, dim3(blocks, 2), dim3(256), 0, st, npix, cw, left,
+            right);
+}
+
 hipError_t launch_prepare(hipStream_t st, const Geometry& g, const float* img,
                           int channels, int stride, ViewBufs v) {
   const dim3 grid((g.W + kBX - 1) / kBX, (g.H + kBY - 1) / kBY);
@@ -2359,13 +2394,13 @@ hipError_t launch_viewbuf_clear_rows(hipStream_t st, const Geometry& g,
   if (n == 0) return hipSuccess;
   const unsigned blocks = (unsigned)((n + 255) / 256);
   PM_LAUNCH(k_viewbuf_clear, dim3(blocks), dim3(256), 0, st, n,
-            vbuf + (size_t)row0 * g.W);
+            vbuf + (size_t)row0 * g.W, (CostWords*)nullptr);
 }
 
 hipError_t launch_viewbuf_clear(hipStream_t st, const Geometry& g,
-                                unsigned long long* vbuf) {
+                                unsigned long long* vbuf, CostWords* cw) {
   const unsigned blocks = (unsigned)((g.npix + 255) / 256);
-  PM_LAUNCH(k_viewbuf_clear, dim3(blocks), dim3(256), 0, st, g.npix, vbuf);
+  PM_LAUNCH(k_viewbuf_clear, dim3(blocks), dim3(256), 0, st, g.npix, vbuf, cw);
 }
 
 template <int kKind, bool kCount, bool kRB, int kRows, int kWX, bool kWin,

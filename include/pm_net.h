@@ -110,8 +110,7 @@ int pm_setup_proposal(pm_ctx* ctx, pm_net* net);
  * at every pixel, the nearest left surface that the view scatter of the
  * seeded left field puts there (the plane the propagate's first view
  * candidate would read), and pmhstereo_init's random plane where none
- * lands, with no cost evaluated (NaN: every propagate re-costs its planes
- * first).  The network's pass over the mirrored pair is saved. */
+ * lands, with no cost evaluated (NaN: the first propagate evaluates it).  The network's pass over the mirrored pair is saved. */
 int pm_setup_proposal_views(pm_ctx* ctx, pm_net* net, int views);
 
 #ifdef __cplusplus
