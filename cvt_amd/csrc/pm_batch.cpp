@@ -63,8 +63,8 @@ struct pm_batch {
   size_t arena_bytes = 0;
   long long nitems = 0;              // tile blocks of all pairs
   pm::BatchShape shape;
-  // the propagate takes wide tiles when every pair's fit a CU, the batch
-  // has enough of them, and the shape is the default or has 8 tile rows
+  // the propagate takes wide tiles when every pair's fit a CU, they pay for
+  // the batch as a whole, and the shape is the default or has 8 tile rows
   bool wide_ok = false;
   bool shape_set = false;            // by pm_batch_set_tuning / _autotune
   long long nwide = 0;               // wide tiles of all pairs
@@ -147,19 +147,20 @@ int check_params(pm_batch* b, const pm_params* p) {
 // descriptor fields that depend on the tile rows: blocks per row and each
 // pair's first block in the batch sequence
 void number_blocks(pm_batch* b) {
-  long long item = 0, wide = 0;
+  long long item = 0, wide = 0, narrow = 0;
   for (pm::BatchPair& P : b->host) {
     P.nbx = (P.g.W + 63) / 64;
     P.item0 = item;
     P.wide0 = wide;
     item += pm::batch_blocks(P.g.W, P.g.H, b->shape.rows);
     wide += pm::wide_tiles(P.g.W, P.g.H);
+    narrow += pm::narrow_pixels(P.g.W, P.g.H);
   }
   b->nitems = item;
   b->nwide = wide;
   b->wide_ok = pm::wide_fits(b->prm.radius, b->prm.cost_kind, b->max_dmax,
                              b->maxW) &&
-               wide >= pm::wide_min_tiles(b->prm.radius);
+               pm::wide_pays(b->prm.radius, wide, narrow);
 }
 
 bool use_wide(const pm_batch* b) {

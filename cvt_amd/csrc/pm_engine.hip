@@ -2425,16 +2425,27 @@ size_t wide_lds_bytes(int R, int cost_kind, float dmax) {
                         window_of(R, dmax, 1).cols);
 }
 
-// The wide tile fits when its window and tiles fit a CU's LDS; it pays
-// (wide_min_tiles) when the image has enough of them: a CU holds one, so an
-// image of 260 tiles takes two rounds with the second nearly empty, and the
-// smaller the patch the less the window saves per tile staged.  Time against
-// the 64 x 4 tiles without a window, plain PatchMatch:
-//   tiles    260   300   350   400   512   650
-//   R = 2   1.11  1.04  1.05  1.01  0.96  0.96
-//   R = 4   1.09  0.99  0.98  0.95  0.91  0.91
-//   R = 5   1.07  0.95  0.96  0.94  0.90  0.90
-int wide_min_tiles(int R) { return R >= 4 ? 300 : 448; }
+// The wide tile pays when the image has enough of them and they cover it
+// without much more padding than 64 x 4 tiles: a CU holds one, so an image of
+// 260 tiles takes two rounds with the second nearly empty, a tile whose
+// second half lies beyond the right border keeps the CU for the first, and
+// the smaller the patch the less the window saves per tile staged.  Time
+// against the 64 x 4 tiles (teams, where those are taken), plain PatchMatch,
+// by padding (wide pixels over narrow ones) and tiles:
+//   padding   1.00                1.06  1.07  1.09  1.11  1.14  1.20  1.33
+//   tiles      260   320   480    700   700   700   700   700   700   700
+//   R = 2     1.11  1.03   .99   1.05  1.02  1.02  1.07  1.10  1.08  1.16
+//   R = 4     1.09   .98   .93    .95   .97   .96  1.02  1.05  1.03  1.16
+//   R = 5     1.07   .97   .91    .95   .97   .96  1.01  1.03  1.02  1.12
+// (widths 640, 1030, 900, 700, 520, 390, 300, 140); R = 4 at 320 tiles and
+// 1.06 to 1.09 1.02 to 1.03.  Uneven batches of 1.03 and 1.06, R = 4: .94 and
+// .98.
+bool wide_pays(int R, long long tiles, long long narrow) {
+  const long long wide = tiles * (kWideCols * kWideRows);
+  const bool tight = 50 * wide <= 51 * narrow;
+  if (tiles < 448) return R >= 4 && tiles >= 300 && tight;
+  return R >= 4 ? 10 * wide <= 11 * narrow : tight;
+}
 
 bool wide_fits(int R, int cost_kind, float dmax, int maxW) {
   return dmax < 4096.0f && maxW < (1 << 23) &&
@@ -2443,6 +2454,10 @@ bool wide_fits(int R, int cost_kind, float dmax, int maxW) {
 long long wide_tiles(int W, int H) {
   return (long long)((W + kWideCols - 1) / kWideCols) *
          ((H + kWideRows - 1) / kWideRows);
+}
+long long narrow_pixels(int W, int H) {
+  return (long long)((W + kTX - 1) / kTX * kTX) *
+         ((H + kTY - 1) / kTY * kTY);
 }
 
 // Teams pay while the image is too small to fill the GPU with one lane per
@@ -2469,12 +2484,6 @@ static hipError_t launch_propagate_kind(hipStream_t st, const Geometry& g,
                                         const PropagateArgs& a,
                                         unsigned long long* counters,
                                         size_t lds_floor) {
-  if (!kRB && !counters && wide_fits(g.R, kKind, a.dmax, g.W) &&
-      wide_tiles(g.W, g.H) >= wide_min_tiles(g.R))
-    return launch_propagate_tile<kKind, false, false, kWideRows,
-                                 kWideCols / kTX, true>(
-        st, g, a, counters, wide_lds_bytes(g.R, kKind, a.dmax),
-        window_of(g.R, a.dmax, a.lr));
   const size_t lds = std::max(
       tile_lds_bytes(g.R, kKind, (kRB ? 2 : 1) * kTX, kTY, 0), lds_floor);
   if (counters)
@@ -2488,6 +2497,12 @@ static hipError_t launch_propagate_kind(hipStream_t st, const Geometry& g,
                                 kTY, 0),
                  lds_floor),
         Window());
+  if (!kRB && wide_fits(g.R, kKind, a.dmax, g.W) &&
+      wide_pays(g.R, wide_tiles(g.W, g.H), narrow_pixels(g.W, g.H)))
+    return launch_propagate_tile<kKind, false, false, kWideRows,
+                                 kWideCols / kTX, true>(
+        st, g, a, counters, wide_lds_bytes(g.R, kKind, a.dmax),
+        window_of(g.R, a.dmax, a.lr));
   return launch_propagate_tile<kKind, false, kRB, kTY, 1, false>(
       st, g, a, counters, lds, Window());
 }
