@@ -63,10 +63,9 @@ struct pm_batch {
   size_t arena_bytes = 0;
   long long nitems = 0;              // tile blocks of all pairs
   pm::BatchShape shape;
-  // the propagate takes wide tiles when every pair's fit a CU, they pay for
-  // the batch as a whole, and the shape is the default or has 8 tile rows
+  // wide tiles: every pair's fit a CU and they pay for the batch as a whole.
+  // The propagate takes them at 8 tile rows, which is the default then.
   bool wide_ok = false;
-  bool shape_set = false;            // by pm_batch_set_tuning / _autotune
   long long nwide = 0;               // wide tiles of all pairs
   float max_dmax = 0.0f;             // largest disparity_max
   bool ran = false;
@@ -163,9 +162,7 @@ void number_blocks(pm_batch* b) {
                pm::wide_pays(b->prm.radius, wide, narrow);
 }
 
-bool use_wide(const pm_batch* b) {
-  return b->wide_ok && (!b->shape_set || b->shape.rows == 8);
-}
+bool use_wide(const pm_batch* b) { return b->wide_ok && b->shape.rows == 8; }
 
 size_t wide_lds(const pm_batch* b) {
   return pm::wide_lds_bytes(b->prm.radius, b->prm.cost_kind, b->max_dmax);
@@ -454,6 +451,10 @@ int pm_batch_create(const pm_params* p, const pm_batch_pair* pairs, int n,
     b->max_dmax = std::max(b->max_dmax, q.disparity_max);
   }
   number_blocks(b);
+  if (b->wide_ok) {
+    b->shape.rows = 8;
+    number_blocks(b);
+  }
   return upload(b);
 }
 
@@ -611,8 +612,7 @@ int pm_batch_set_tuning(pm_batch* b, const pm_batch_tuning* t) {
   int rc;
   if ((rc = allow_shape(b, t->tile_rows))) return rc;
   if (t->tile_rows != b->shape.rows ||
-      t->workgroups != b->shape.workgroups || !b->shape_set) {
-    b->shape_set = true;
+      t->workgroups != b->shape.workgroups) {
     b->shape.rows = t->tile_rows;
     b->shape.workgroups = t->workgroups;
     b->tuned_ms = 0.0f;
@@ -641,6 +641,7 @@ int pm_batch_autotune(pm_batch* b, int reps, pm_batch_tuning* table,
                                   &resident) != hipSuccess ||
         resident < 1)
       continue;
+    if (rows == 8 && b->wide_ok) resident = 1;  // a wide tile fills a CU
     const int full = cus * resident;
     for (int wg : {full, 2 * full, 0}) {
       pm_batch_tuning t{};

@@ -54,7 +54,8 @@ typedef struct pm_batch_pair {
 /* Launch shape of the persistent tile kernels. */
 typedef struct pm_batch_tuning {
     int tile_rows;       /* 2, 4 or 8: work-groups of 64 x tile_rows pixels (8:
-                            the propagate's are 128 x 8 where that fits) */
+                            the propagate's are 128 x 8 where that fits and
+                            pays, the default then; else the default is 4) */
     int workgroups;      /* persistent grid; 0 = one work-group per tile */
     float ms;            /* pm_batch_autotune: time of one view's propagate
                             over the batch with this shape (ms); else 0 */
