@@ -2473,10 +2473,23 @@ long long narrow_pixels(int W, int H) {
 //                (1.18)(1.17) (.88) (.94) (.79) (.85) (.75)
 //   560 x 416     1.43  1.41  1.06  1.13   .94  1.01   .90
 //                (1.21)(1.16) (.87) (.93) (.77) (.83) (.73)
-static bool team_pays(int R, int W, int H) {
+// Beside PM-Huber smoothing, which takes CUs itself, the line lies lower.
+// depthMap (disparityMap is alike), 4 iterations, teams against without:
+//   pixels      30000  50700  76800  108300  145200  187500
+//   R = 1         .92    .96   1.01    1.06
+//   R = 2         .81    .92   1.00
+//   R = 3         .63    .78    .87     .97     .98    1.08
+//   R = 4         .59    .76    .90    1.02    1.03    1.15
+//   R = 5         .46    .67    .79     .90     .90    1.02
+// and the work-groups ask for no more LDS than they use: with the floor that
+// makes room for the smoothing beside 64 x 4 tiles, 50700 pixels take 2 to 9
+// % more time, 187500 pixels 7 %.
+static bool team_pays(int R, int W, int H, bool smoothing) {
   const long long taps = 2 * R + 1;
   const long long slots = (taps + kTeamLanes - 1) / kTeamLanes * kTeamLanes;
-  return (long long)W * H * slots <= taps * (R < 3 ? 150000 : 262144);
+  const long long line = smoothing ? (R < 3 ? 90000 : 163840)
+                                   : (R < 3 ? 150000 : 262144);
+  return (long long)W * H * slots <= taps * line;
 }
 
 template <int kKind, bool kRB>
@@ -2490,12 +2503,10 @@ static hipError_t launch_propagate_kind(hipStream_t st, const Geometry& g,
     return launch_propagate_tile<kKind, true, kRB, kTY, 1, false>(
         st, g, a, counters, lds, Window());
   // (a radius whose 64 x 4 tile does not fit is refused below)
-  if (lds <= kLdsPerCu && team_pays(g.R, g.W, g.H))
+  if (lds <= kLdsPerCu && team_pays(g.R, g.W, g.H, a.smooth != nullptr))
     return launch_propagate_tile<kKind, false, kRB, kTY, 1, false, kTeamLanes>(
         st, g, a, counters,
-        std::max(tile_lds_bytes(g.R, kKind, (kRB ? 2 : 1) * kTX / kTeamLanes,
-                                kTY, 0),
-                 lds_floor),
+        tile_lds_bytes(g.R, kKind, (kRB ? 2 : 1) * kTX / kTeamLanes, kTY, 0),
         Window());
   if (!kRB && wide_fits(g.R, kKind, a.dmax, g.W) &&
       wide_pays(g.R, wide_tiles(g.W, g.H), narrow_pixels(g.W, g.H)))
