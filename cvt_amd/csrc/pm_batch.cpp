@@ -159,7 +159,7 @@ void number_blocks(pm_batch* b) {
   b->nwide = wide;
   b->wide_ok = pm::wide_fits(b->prm.radius, b->prm.cost_kind, b->max_dmax,
                              b->maxW) &&
-               pm::wide_pays(b->prm.radius, wide, narrow);
+               pm::wide_pays(b->prm.radius, wide, narrow, true);
 }
 
 bool use_wide(const pm_batch* b) { return b->wide_ok && b->shape.rows == 8; }

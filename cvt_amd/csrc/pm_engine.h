@@ -175,12 +175,13 @@ hipError_t launch_propagate(hipStream_t st, const Geometry& g,
 // The propagate's wide tile (pm_engine.hip): its LDS at a patch radius, cost
 // kind and disparity range, whether that fits a CU, the tiles of an image,
 // the pixels of the 64 x 4 tiles that cover it, and whether the wide ones are
-// the better cover (both may be sums over images).
+// the better cover (both may be sums over images; alone: of a launch that no
+// other work overlaps).
 size_t wide_lds_bytes(int R, int cost_kind, float dmax);
 bool wide_fits(int R, int cost_kind, float dmax, int maxW);
 long long wide_tiles(int W, int H);
 long long narrow_pixels(int W, int H);
-bool wide_pays(int R, long long tiles, long long narrow);
+bool wide_pays(int R, long long tiles, long long narrow, bool alone);
 
 hipError_t launch_scatter(hipStream_t st, const Geometry& g,
                           const float4* states, int lr,

@@ -101,6 +101,7 @@ __host__ __device__ __forceinline__ size_t tile_lds_bytes(int R, int kind,
 // CU, with the window of the other view's gradients in LDS.
 constexpr int kWideCols = 128, kWideRows = 8;
 constexpr size_t kLdsPerCu = 160 * 1024;
+constexpr int kCus = 256;
 
 // The window of a wide tile: x' = x - d (left view) or x + d (right), d in
 // [0, dmax], and room on both sides for the patch, KLT's neighbours and
@@ -1844,11 +1845,12 @@ __device__ __forceinline__ void propagate_block(
   }
 }
 
-// The single-image launch: one tile block per work-group.
+// The single-image launch: one tile block per work-group.  kEu: wavefronts
+// per SIMD the kernel is built for (see saves_a_round).
 template <int kKind, bool kCount, bool kRB, int kRows, int kWX, bool kWin,
-          int kTeam>
+          int kTeam, int kEu>
 __global__ void __launch_bounds__(64 * kWX * kRows)
-__attribute__((amdgpu_waves_per_eu(4, 4)))
+__attribute__((amdgpu_waves_per_eu(kEu, kEu)))
 k_propagate(Geometry g, PropagateArgs a, unsigned long long* counters,
             Window win) {
   extern __shared__ float4 smem[];
@@ -2176,9 +2178,9 @@ __device__ __forceinline__ PropagateArgs batch_args(const BatchPair& P,
   return a;
 }
 
-template <int kKind, int kRows>
+template <int kKind, int kRows, int kEu>
 __global__ void __launch_bounds__(64 * kRows)
-__attribute__((amdgpu_waves_per_eu(4, 4)))
+__attribute__((amdgpu_waves_per_eu(kEu, kEu)))
 k_propagate_batch(const BatchPair* __restrict__ pairs, int npairs,
                   long long nitems, int view, int cur, int iter) {
   extern __shared__ float4 smem[];
@@ -2404,7 +2406,7 @@ hipError_t launch_viewbuf_clear(hipStream_t st, const Geometry& g,
 }
 
 template <int kKind, bool kCount, bool kRB, int kRows, int kWX, bool kWin,
-          int kTeam = 1>
+          int kTeam = 1, int kEu = 4>
 static hipError_t launch_propagate_tile(hipStream_t st, const Geometry& g,
                                         const PropagateArgs& a,
                                         unsigned long long* counters,
@@ -2413,11 +2415,30 @@ static hipError_t launch_propagate_tile(hipStream_t st, const Geometry& g,
   const int rows = g.row_end() - g.band0 * kBandRows;
   const dim3 grid((unsigned)((g.W + cols - 1) / cols),
                   (unsigned)((rows + kRows - 1) / kRows));
-  const hipError_t e =
-      allow_lds(k_propagate<kKind, kCount, kRB, kRows, kWX, kWin, kTeam>, lds);
+  constexpr auto kernel =
+      k_propagate<kKind, kCount, kRB, kRows, kWX, kWin, kTeam, kEu>;
+  const hipError_t e = allow_lds(kernel, lds);
   if (e != hipSuccess) return e;
-  PM_LAUNCH((k_propagate<kKind, kCount, kRB, kRows, kWX, kWin, kTeam>), grid,
-            dim3(kTX * kWX, kRows), lds, st, g, a, counters, win);
+  PM_LAUNCH(kernel, grid, dim3(kTX * kWX, kRows), lds, st, g, a, counters, win);
+}
+
+// Five wavefronts per SIMD, at 96 registers and some spills, are 1 to 7 %
+// slower than four while either fills the GPU, but a launch with nothing
+// beside it (a batch's, a red-black pass) that is a little more than one or
+// a few rounds of four takes a round less with five.  Batches by work-groups
+// of 64 x 4 pixels (1024 to a round of four, 1280 to one of five), the time
+// with four and with five against a kernel of five whose candidates were
+// unrolled:
+//   900  1050  1092  1200  1272  1320  1800  2000  2100  2208  2400  3180  3600
+//   .94   .82   .98  1.15  1.08   .98   .92   .88  1.02  1.03   .93   .97   .92
+//   .95   .95   .95   .94   .95   .94   .99   .95   .93   .94   .94   .95   .94
+static bool saves_a_round(long long workgroups, int waves, size_t lds) {
+  if (20 % waves || 20 / waves * lds > kLdsPerCu) return false;
+  const long long four = 4 * kCus * 4, five = 5 * kCus * 4;
+  const long long n = workgroups * waves;
+  const long long over = n - 128;  // 3 % more fit into a round's end
+  return (over + four - 1) / four > (n + five - 1) / five &&
+         (over - 1) % four < 1920;
 }
 
 size_t wide_lds_bytes(int R, int cost_kind, float dmax) {
@@ -2440,8 +2461,21 @@ size_t wide_lds_bytes(int R, int cost_kind, float dmax) {
 // (widths 640, 1030, 900, 700, 520, 390, 300, 140); R = 4 at 320 tiles and
 // 1.06 to 1.09 1.02 to 1.03.  Uneven batches of 1.03 and 1.06, R = 4: .94 and
 // .98.
-bool wide_pays(int R, long long tiles, long long narrow) {
+//   A launch with nothing beside it (alone: a batch's; an image's bands and
+// iterations overlap) also ends with a round that has to be half full, the
+// sooner the fewer rounds there are.  Of 110 batches of 128 to 896 columns,
+// the wide tiles' time against the better of the others at tiles
+//   250-325    1.0-1.5    (one round of 256, almost or just over)
+//   330-488    .74-1.0
+//   490-610    1.0-1.25
+//   620-750     .83-1.0
+//   756-836     .94-1.1
+//   880-1000    .85-.97
+//   1064-1130   .95-1.0    (from there on .88-.98)
+bool wide_pays(int R, long long tiles, long long narrow, bool alone) {
   const long long wide = tiles * (kWideCols * kWideRows);
+  if (alone && tiles < 1130 && (tiles + 24 + kCus - 1) % kCus + 1 < 130)
+    return false;
   const bool tight = 50 * wide <= 51 * narrow;
   if (tiles < 448) return R >= 4 && tiles >= 300 && tight;
   return R >= 4 ? 10 * wide <= 11 * narrow : tight;
@@ -2509,11 +2543,20 @@ static hipError_t launch_propagate_kind(hipStream_t st, const Geometry& g,
         tile_lds_bytes(g.R, kKind, (kRB ? 2 : 1) * kTX / kTeamLanes, kTY, 0),
         Window());
   if (!kRB && wide_fits(g.R, kKind, a.dmax, g.W) &&
-      wide_pays(g.R, wide_tiles(g.W, g.H), narrow_pixels(g.W, g.H)))
+      wide_pays(g.R, wide_tiles(g.W, g.H), narrow_pixels(g.W, g.H), false))
     return launch_propagate_tile<kKind, false, false, kWideRows,
                                  kWideCols / kTX, true>(
         st, g, a, counters, wide_lds_bytes(g.R, kKind, a.dmax),
         window_of(g.R, a.dmax, a.lr));
+  // a red-black pass only in five's first round: 640 x 960 1.00 with four,
+  // .96 with five (R = 4); 1280 x 960 .92 and .95
+  const long long blocks = (long long)((g.W + 2 * kTX - 1) / (2 * kTX)) *
+                           ((g.H + kTY - 1) / kTY);
+  if (kRB && !lds_floor && blocks <= 5 * kCus &&
+      saves_a_round(blocks, kTY, lds))
+    return launch_propagate_tile<kKind, false, kRB, kTY, 1, false, 1,
+                                 kRB ? 5 : 4>(st, g, a, counters, lds,
+                                              Window());
   return launch_propagate_tile<kKind, false, kRB, kTY, 1, false>(
       st, g, a, counters, lds, Window());
 }
@@ -2694,16 +2737,30 @@ hipError_t launch_init_batch(hipStream_t st, const BatchPair* pairs,
                                       shape);
 }
 
+template <int kKind, int kRows, int kEu>
+static hipError_t propagate_batch_built(hipStream_t st,
+                                        const BatchPair* pairs, int npairs,
+                                        long long nitems, int view, int cur,
+                                        int iter, size_t lds,
+                                        BatchShape shape) {
+  constexpr auto kernel = k_propagate_batch<kKind, kRows, kEu>;
+  const hipError_t e = allow_lds(kernel, lds);
+  if (e != hipSuccess) return e;
+  PM_LAUNCH(kernel, dim3(batch_tile_grid(nitems, shape)), dim3(kTX, kRows),
+            lds, st, pairs, npairs, nitems, view, cur, iter);
+}
+
+// (8 rows: five per SIMD would be two and a half work-groups a CU)
 template <int kKind, int kRows>
 static hipError_t propagate_batch_rows(hipStream_t st, const BatchPair* pairs,
                                        int npairs, long long nitems, int view,
                                        int cur, int iter, size_t lds,
                                        BatchShape shape) {
-  const hipError_t e = allow_lds(k_propagate_batch<kKind, kRows>, lds);
-  if (e != hipSuccess) return e;
-  PM_LAUNCH((k_propagate_batch<kKind, kRows>),
-            dim3(batch_tile_grid(nitems, shape)), dim3(kTX, kRows), lds, st,
-            pairs, npairs, nitems, view, cur, iter);
+  if (kRows < 8 && shape.workgroups == 0 && saves_a_round(nitems, kRows, lds))
+    return propagate_batch_built<kKind, kRows, kRows < 8 ? 5 : 4>(
+        st, pairs, npairs, nitems, view, cur, iter, lds, shape);
+  return propagate_batch_built<kKind, kRows, 4>(
+      st, pairs, npairs, nitems, view, cur, iter, lds, shape);
 }
 
 template <int kKind>
@@ -2766,10 +2823,13 @@ hipError_t batch_allow_wide(int cost_kind, size_t lds) {
 
 template <int kKind, int kRows>
 static hipError_t resident_rows(size_t lds, int* out) {
-  hipError_t e = allow_lds(k_propagate_batch<kKind, kRows>, lds);
+  hipError_t e = hipSuccess;
+  if (kRows < 8)  // before a capture, as the one the occupancy is asked of
+    e = allow_lds(k_propagate_batch<kKind, kRows, kRows < 8 ? 5 : 4>, lds);
+  if (e == hipSuccess) e = allow_lds(k_propagate_batch<kKind, kRows, 4>, lds);
   if (e != hipSuccess) return e;
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      out, k_propagate_batch<kKind, kRows>, kTX * kRows, lds);
+      out, k_propagate_batch<kKind, kRows, 4>, kTX * kRows, lds);
 }
 
 hipError_t batch_resident_per_cu(int cost_kind, int rows, size_t lds,
