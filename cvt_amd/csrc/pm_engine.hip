@@ -2548,15 +2548,18 @@ static hipError_t launch_propagate_kind(hipStream_t st, const Geometry& g,
                                  kWideCols / kTX, true>(
         st, g, a, counters, wide_lds_bytes(g.R, kKind, a.dmax),
         window_of(g.R, a.dmax, a.lr));
-  // a red-black pass only in five's first round: 640 x 960 1.00 with four,
-  // .96 with five (R = 4); 1280 x 960 .92 and .95
+  // The build for five: beside smoothing, three work-groups a CU whichever it
+  // is, from radius 4 on for the registers it leaves (radius 5, 620 x 465:
+  // depthMap 20.5 ms with the build for four, 18.3 with it; 1 to 2 % more where
+  // the smoothing fits beside either, as it always did at radius 2 and 3), and
+  // in red-black's passes, in its first round only (640 x 960, R = 4: 1.00 with
+  // four, .96 with five; 1280 x 960 .92 and .95).
   const long long blocks = (long long)((g.W + 2 * kTX - 1) / (2 * kTX)) *
                            ((g.H + kTY - 1) / kTY);
-  if (kRB && !lds_floor && blocks <= 5 * kCus &&
-      saves_a_round(blocks, kTY, lds))
-    return launch_propagate_tile<kKind, false, kRB, kTY, 1, false, 1,
-                                 kRB ? 5 : 4>(st, g, a, counters, lds,
-                                              Window());
+  if (a.smooth ? g.R >= 4
+               : kRB && blocks <= 5 * kCus && saves_a_round(blocks, kTY, lds))
+    return launch_propagate_tile<kKind, false, kRB, kTY, 1, false, 1, 5>(
+        st, g, a, counters, lds, Window());
   return launch_propagate_tile<kKind, false, kRB, kTY, 1, false>(
       st, g, a, counters, lds, Window());
 }

@@ -1,6 +1,7 @@
 """Teams of four lanes per pixel beside PM-Huber smoothing, right below and
-right above their line there (pm_engine.hip, team_pays), bit for bit against
-the oracle."""
+right above their line there (pm_engine.hip, team_pays), where radius 5 takes
+the propagate built for five wavefronts and radius 1 the one for four, bit for
+bit against the oracle."""
 import pytest
 
 import cvt_amd
