@@ -726,15 +726,17 @@ int postprocess(pm_ctx* c, int pp, float maxdispdiff, float maxdeg,
 
 // With PM_SMOOTH_HUBER each view's smoothing runs beside the other view's
 // propagate.  Propagate work-groups of 64 x 4 pixels fill a CU's VGPRs (four
-// per CU at 128 VGPRs) and leave no room for a k_rof_steps work-group, which
-// then gets a CU only when propagate work-groups retire.  Asking for just
-// over a quarter of a CU's LDS per propagate work-group caps them at three
-// per CU and leaves LDS and VGPRs (3 x 128 + 120 of 512 per lane) for one
-// smoothing work-group beside them.  Measured on the 720p pair with a build
-// of 96 VGPRs: 8 coupled iterations 64.4 -> 61.5 ms.  Plain PatchMatch keeps
-// the CU to itself (three per CU would cost it 4 %).  The wide tile fills a
-// CU with one work-group whatever it asks for and takes no floor: its
-// smoothing runs on the CUs that the last tiles of a half launch leave.
+// per CU at 128 VGPRs, five at 96, which the propagate takes here from radius
+// 4 on) and leave no room for a k_rof_steps work-group, which then gets a CU
+// only when propagate work-groups retire.  Asking for just over a quarter of
+// a CU's LDS per propagate work-group caps them at three per CU and leaves
+// LDS and VGPRs (3 x 128 + 120 of 512 per lane) for one smoothing work-group
+// beside them.  Measured on the 720p pair with a build of 96 VGPRs: 8 coupled
+// iterations 64.4 -> 61.5 ms.  Plain PatchMatch keeps the CU to itself (three
+// per CU would cost it 4 %).  Teams take no floor (team_pays), and neither
+// does the wide tile, which fills a CU with one work-group whatever it asks
+// for: its smoothing runs on the CUs that the last tiles of a half launch
+// leave.
 // The floor is kept only when three such work-groups and one k_rof_steps
 // work-group fit the CU's LDS, allocated in 512-byte granules.
 int share_cus_with_smoothing(pm_ctx* c) {

@@ -164,9 +164,9 @@ struct PropagateArgs {
 constexpr int kFlatCosts = 2;
 
 // counters (optional, 2 x u64): cost taps and KLT taps evaluated, counted
-// with the reference's per-tap early exit.  lds_floor: the work-groups ask
-// for at least this much LDS (only the tile's share is used), which caps
-// how many share a CU.
+// with the reference's per-tap early exit.  lds_floor: the 64 x 4 tiles'
+// work-groups ask for at least this much LDS (only the tile's share is used),
+// which caps how many share a CU.
 hipError_t launch_propagate(hipStream_t st, const Geometry& g,
                             const PropagateArgs& a,
                             unsigned long long* counters = nullptr,

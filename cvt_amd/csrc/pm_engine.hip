@@ -1270,7 +1270,7 @@ __device__ __forceinline__ float4 klt_team(const Lane& L, float4 s) {
       const float rowb = s.y * py;  // transform(), b y per row
       const float4* __restrict__ srow = L.tex2 + (size_t)qy * L.TS;
       const LdsRow trow = L.trow0 + (dy + R) * L.TW;
-        const float jb = L.sub == 0 ? 0.0f : (L.sub == 1 ? py : 1.0f);
+      const float jb = L.sub == 0 ? 0.0f : (L.sub == 1 ? py : 1.0f);
       const float ab = L.sub == 3 ? py : 0.0f;
       const float bb = L.sub == 0 ? 0.0f : (L.sub == 2 ? 1.0f : py);
       const float cB = L.sub == 0 ? py : 1.0f;              // py 1
@@ -2306,7 +2306,7 @@ static hipError_t allow_lds(K kernel, size_t bytes) {
 
 #define PM_LAUNCH_TILE(kernel, kind, g, st, ...)                        \
   do {                                                                  \
-    const size_t lds_ = tile_lds_bytes((g).R, kind, kTX, kTY, 0);                   \
+    const size_t lds_ = tile_lds_bytes((g).R, kind, kTX, kTY, 0);       \
     hipError_t e_ = allow_lds(kernel, lds_);                            \
     if (e_ != hipSuccess) return e_;                                    \
     PM_LAUNCH(kernel, grid_for(g), kBlockTile, lds_, st,                \
@@ -2425,10 +2425,10 @@ static hipError_t launch_propagate_tile(hipStream_t st, const Geometry& g,
 // Five wavefronts per SIMD, at 96 registers and some spills, are 1 to 7 %
 // slower than four while either fills the GPU, but a launch with nothing
 // beside it (a batch's, a red-black pass) that is a little more than one or
-// a few rounds of four takes a round less with five.  Batches by work-groups
-// of 64 x 4 pixels (1024 to a round of four, 1280 to one of five), the time
-// with four and with five against a kernel of five whose candidates were
-// unrolled:
+// a few rounds of four takes a round less with five (from six rounds on it is
+// all one).  Batches by work-groups of 64 x 4 pixels (1024 to a round of four,
+// 1280 to one of five), the time with four and with five against a kernel of
+// five whose candidates were unrolled:
 //   900  1050  1092  1200  1272  1320  1800  2000  2100  2208  2400  3180  3600
 //   .94   .82   .98  1.15  1.08   .98   .92   .88  1.02  1.03   .93   .97   .92
 //   .95   .95   .95   .94   .95   .94   .99   .95   .93   .94   .94   .95   .94
@@ -2437,7 +2437,8 @@ static bool saves_a_round(long long workgroups, int waves, size_t lds) {
   const long long four = 4 * kCus * 4, five = 5 * kCus * 4;
   const long long n = workgroups * waves;
   const long long over = n - 128;  // 3 % more fit into a round's end
-  return (over + four - 1) / four > (n + five - 1) / five &&
+  return n < 6 * four &&
+         (over + four - 1) / four > (n + five - 1) / five &&
          (over - 1) % four < 1920;
 }
 
