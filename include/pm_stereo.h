@@ -180,7 +180,7 @@ int pm_setup_prior(pm_ctx* ctx, const float* disparity, const float* normals);
  * context's stream before it returns, so the call stays ordered on that
  * stream like any other.  Consecutive propagates overlap only within one
  * call, so run the iterations as one call where possible (8 iterations of
- * a 720p pair: 44.8 ms as one call, 52.1 ms as eight calls of one).  With
+ * a 720p pair: 45.1 ms as one call, 52.3 ms as eight calls of one).  With
  * PM_SMOOTH_NONE the call can be recorded by stream capture on the
  * context's stream; with PM_SMOOTH_HUBER or PM_SMOOTH_DEPTHMAP a
  * capturing stream gets PM_ERR_ARG before anything is queued. */
